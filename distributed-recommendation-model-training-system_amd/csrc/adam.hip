@@ -420,6 +420,136 @@ __device__ void FinishBlock(const RowStats& st, Control* ctrl, Bounds* bounds, b
 }
 
 // ---------------------------------------------------------------------------
+// Long rows of the drivers below: one row's references summed by a whole block.
+// A group's own loop keeps four gradient rows in flight, so a row of thousands
+// of references would hold its group (and the launch) for a memory latency per
+// four of them.  Here the block's threads load a tile of references together
+// (kLongLoads elements a thread: 8 KiB of floats for the vector shapes), scale
+// them and stage the products in LDS as [reference][column]; thread c then
+// adds column c of the tile in reference order while the next tile's rows and
+// the reference words of the one after it are already on their way.  The sum
+// is the group loop's, bit for bit: acc = acc + src * scale, in order, from +0.
+// A tile takes about 1.3 us, the latency of its rows.  Six tables of dims 10 to
+// 300, 10,600 references each, their longest rows ~1,000: the reduce kernels
+// 1,807 -> 224 us, with every class in one launch.
+constexpr uint32_t kBlockRowRefs = 32;   // rows with more references are summed by the block
+constexpr uint32_t kLongTile = 8192;     // floats of a staged tile
+
+// Waits for this wave's LDS accesses, then for the block's other waves: unlike
+// __syncthreads it leaves global loads in flight.
+__device__ __forceinline__ void LdsBarrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The references of one row of the sorted array: Load reads reference i's
+// word, Source decodes it to column `at` of its gradient row (`safe` and ok
+// false when it names none of the push) and scale.
+struct SortedRefs {
+  typedef uint64_t Word;
+  const uint64_t* rs;
+  const float* const* grad;
+  const uint64_t* rows;  // gradient rows per feature
+  const float* safe;
+  uint32_t features, dim;
+  __device__ __forceinline__ Word Load(uint32_t i) const { return rs[i]; }
+  __device__ __forceinline__ const float* Source(Word w, uint32_t at, float& scale, bool& ok) const {
+    const RefParts rp = SplitRef(w);
+    const uint32_t f = min(rp.feature, features - 1);
+    const bool in = RefInRange(rp, features, rows[f]);
+    if (!in) ok = false;
+    scale = __uint_as_float(uint32_t(w >> 32));
+    return in ? grad[f] + uint64_t(rp.row) * dim + at : safe;
+  }
+};
+
+// The references of one row of a CSR packet (already range-checked by the
+// gradient scan).
+struct CsrRefs {
+  struct Word { uint64_t row; float scale; };
+  const uint64_t* sources;
+  const float* scales;
+  const float* src;
+  uint32_t dim;
+  __device__ __forceinline__ Word Load(uint32_t i) const { return Word{sources[i], scales[i]}; }
+  __device__ __forceinline__ const float* Source(Word w, uint32_t at, float& scale, bool&) const {
+    scale = w.scale;
+    return src + w.row * dim + at;
+  }
+};
+
+// `acc` plus references [0, count) of column c0 + threadIdx.x (`acc` when that
+// lies past the dimension; vector shapes: c0 = 0, dim <= 256).  `ok` turns
+// false in any thread that met a reference of no gradient row.  Called by the whole
+// block; `tile` holds kLongTile floats.
+template <bool kVec, class Refs>
+__device__ __forceinline__ float BlockRowSum(float* tile, const Refs& refs, uint32_t count, uint32_t dim,
+                                             uint32_t c0, float acc, bool& ok) {
+  constexpr uint32_t kLongLoads = kVec ? 8 : 16;
+  const uint32_t width = kVec ? dim / 4 : min(dim - c0, kBlock);  // elements of a reference
+  uint32_t log2g = 2;                                             // lanes of a reference
+  while ((1u << log2g) < width) ++log2g;
+  const uint32_t pitch = kVec ? dim : width, cols = pitch;
+  const uint32_t per_step = kBlock >> log2g, tile_refs = kLongLoads * per_step;
+  const uint32_t sub = threadIdx.x >> log2g, e = threadIdx.x & ((1u << log2g) - 1);
+  const bool active = e < width;
+  const uint32_t at = active ? (kVec ? e * 4 : c0 + e) : (kVec ? 0u : c0);
+  float4 x[kLongLoads];
+  float scale[kLongLoads];
+  typename Refs::Word w[kLongLoads];
+  // References past the row's end repeat its last one and are not added.
+  auto load_words = [&](uint32_t base) {
+#pragma unroll
+    for (uint32_t k = 0; k < kLongLoads; ++k) w[k] = refs.Load(min(base + k * per_step + sub, count - 1));
+  };
+  auto load_rows = [&]() {
+    const float* src[kLongLoads];
+#pragma unroll
+    for (uint32_t k = 0; k < kLongLoads; ++k) src[k] = refs.Source(w[k], at, scale[k], ok);
+#pragma unroll
+    for (uint32_t k = 0; k < kLongLoads; ++k) {
+      if constexpr (kVec) x[k] = Load4(src[k]);
+      else x[k].x = LoadF(src[k]);
+    }
+  };
+  load_words(0);
+  load_rows();
+  load_words(tile_refs);
+  for (uint32_t base = 0; base < count; base += tile_refs) {
+    LdsBarrier();  // the tile before has been added
+    if (active) {
+#pragma unroll
+      for (uint32_t k = 0; k < kLongLoads; ++k) {
+        float* to = tile + (k * per_step + sub) * pitch + (kVec ? e * 4 : e);
+        if constexpr (kVec)
+          *reinterpret_cast<float4*>(to) =
+              make_float4(x[k].x * scale[k], x[k].y * scale[k], x[k].z * scale[k], x[k].w * scale[k]);
+        else
+          *to = x[k].x * scale[k];
+      }
+    }
+    load_rows();
+    load_words(base + 2 * tile_refs);
+    LdsBarrier();
+    if (threadIdx.x < cols) {
+      const uint32_t n = min(tile_refs, count - base);
+      const float* col = tile + threadIdx.x;
+      uint32_t r = 0;
+      for (; r + 16 <= n; r += 16) {
+        float v[16];
+#pragma unroll
+        for (uint32_t k = 0; k < 16; ++k) v[k] = col[(r + k) * pitch];
+#pragma unroll
+        for (uint32_t k = 0; k < 16; ++k) acc = acc + v[k];
+      }
+      for (; r < n; ++r) acc = acc + col[r * pitch];
+    }
+  }
+  return acc;
+}
+
+// ---------------------------------------------------------------------------
 // Sorted driver: segments are runs of equal keys in the sorted key array.
 struct FusedArgs {
   TableDesc t[EPS_HIP_MAX_TABLES];   // by key index
@@ -434,135 +564,206 @@ struct FusedArgs {
   Control* ctrl;
   Bounds* bounds;
   GuardScalars gs;
-  uint32_t row_bits, cls, cls_end, log2g, ppb, vblocks, role, reduce, tables, features;  // classes [cls, cls_end)
+  uint32_t row_bits, cls, cls_end, vblocks, role, tables, features;  // classes [cls, cls_end)
   uint32_t n;  // occurrences of the push (sorted positions, occurrence indices)
+  uint32_t class_block[kClasses + 1];  // SortedReduceKernel: first block of each class (and the total)
 };
 static_assert(sizeof(FusedArgs) <= 4096, "update arguments fit the kernel-argument segment");
 
-template <bool kGeneric>
-__global__ void __launch_bounds__(kBlock) SortedUpdateKernel(FusedArgs a) {
-  __shared__ TableDesc s_t[EPS_HIP_MAX_TABLES];
-  __shared__ const float* s_grad[EPS_HIP_MAX_FEATURES];
-  __shared__ uint32_t s_heads[kBlock];
-  __shared__ uint32_t s_wave_heads[4];
-  __shared__ uint32_t s_mode;
-  __shared__ uint64_t s_rows[EPS_HIP_MAX_FEATURES];  // gradient rows per feature
-  CopyWords(s_t, a.t, sizeof(a.t));
-  CopyWords(s_grad, a.grad, sizeof(a.grad));
-  CopyWords(s_rows, a.grad_rows, sizeof(a.grad_rows));
-  Control* ctrl = a.ctrl;
-  bool write = true;
-  if (!a.reduce && !LaunchGate(ctrl, s_t, a.gs, a.role, &s_mode, write)) return;
-  // The classes' sorted positions, from the workspace, kept inside the push's.
-  const uint32_t first = ctrl->class_start[a.cls], last = ctrl->class_start[a.cls_end];
-  const uint32_t end = min(last, a.n), start = min(first, end);
-  const uint32_t G = kGeneric ? kWave : (1u << a.log2g);
+struct SortedShared {
+  TableDesc t[EPS_HIP_MAX_TABLES];
+  const float* grad[EPS_HIP_MAX_FEATURES];
+  uint64_t rows[EPS_HIP_MAX_FEATURES];  // gradient rows per feature
+  uint32_t heads[kBlock];
+  uint32_t wave_heads[kBlock / kWave];
+  uint32_t mode, bad;
+  __align__(16) float tile[kLongTile];
+};
+
+// The rows whose first position lies in the windows of `ppb` positions that
+// virtual blocks vb, vb + step, ... < vblocks of the positions [start, end)
+// own.  A row of up to kBlockRowRefs references takes one group of 2^log2g
+// lanes (kGeneric: a wavefront over scalar columns), a longer one the block.
+template <bool kGeneric, bool kReduce>
+__device__ __forceinline__ void SortedRows(const FusedArgs& a, SortedShared& sh, uint32_t start, uint32_t end,
+                                           uint32_t log2g, uint32_t ppb, uint32_t vb, uint32_t step,
+                                           uint32_t vblocks, bool write, RowStats& st) {
+  const uint32_t G = kGeneric ? kWave : (1u << log2g);
   const uint32_t lig = threadIdx.x & (G - 1);
   const uint32_t gid = threadIdx.x / G, ngroups = kBlock / G;
   const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  RowStats st;
-  __syncthreads();
-  for (uint32_t vb = blockIdx.x; vb < a.vblocks; vb += gridDim.x) {
-    const uint32_t p0 = start + vb * a.ppb;
+  const float* safe = reinterpret_cast<const float*>(a.ctrl);
+  for (; vb < vblocks; vb += step) {
+    const uint32_t p0 = start + vb * ppb;
     if (p0 >= end) break;  // uniform: later virtual blocks are further right
-    const uint32_t p1 = min(p0 + a.ppb, end);
+    const uint32_t p1 = min(p0 + ppb, end);
     // Head positions of this block's range, in order.
     const uint32_t p = p0 + threadIdx.x;
-    const bool head = threadIdx.x < a.ppb && p < p1 && (p == start || a.keys[p] != a.keys[p - 1]);
+    const bool head = threadIdx.x < ppb && p < p1 && (p == start || a.keys[p] != a.keys[p - 1]);
     const uint64_t ballot = __ballot(head);
-    if (lane == 0) s_wave_heads[wave] = uint32_t(__popcll(ballot));
+    if (lane == 0) sh.wave_heads[wave] = uint32_t(__popcll(ballot));
+    if (threadIdx.x == 0) sh.bad = 0;
     __syncthreads();
     uint32_t before = 0;
-    for (uint32_t w = 0; w < wave; ++w) before += s_wave_heads[w];
-    const uint32_t nheads = s_wave_heads[0] + s_wave_heads[1] + s_wave_heads[2] + s_wave_heads[3];
-    if (head) s_heads[before + uint32_t(__popcll(ballot & ((1ull << lane) - 1)))] = p;
+    for (uint32_t w = 0; w < wave; ++w) before += sh.wave_heads[w];
+    const uint32_t nheads = sh.wave_heads[0] + sh.wave_heads[1] + sh.wave_heads[2] + sh.wave_heads[3];
+    if (head) sh.heads[before + uint32_t(__popcll(ballot & ((1ull << lane) - 1)))] = p;
     __syncthreads();
+    if (!nheads) continue;
+    const uint32_t last_end = SegmentEndSearch(a.keys, p1, end, a.keys[p1 - 1]);
+    // What row h is: a key or reference naming nothing of the push (a damaged
+    // workspace) is not used as an address: its loads read zero and the row is
+    // not written.  The reference checks see the same words in every lane.
+    struct Row { uint32_t sb, se; KeyParts kp; bool ok; uint64_t u; };
+    auto row_of = [&](uint32_t h) {
+      Row r;
+      r.sb = sh.heads[h];
+      r.se = h + 1 < nheads ? sh.heads[h + 1] : last_end;
+      r.kp = SplitKey(a.keys[r.sb], a.row_bits);
+      r.ok = KeyInRange(r.kp, a.tables, sh.t[min(r.kp.table, a.tables - 1)].rows);
+      r.u = 0;
+      if (kReduce) {
+        const uint32_t occ = a.vals[r.sb];
+        r.ok = r.ok && occ < a.n;
+        r.u = r.ok ? a.occ2u[occ] : 0;
+      }
+      return r;
+    };
     for (uint32_t h = gid; h < nheads; h += ngroups) {
-      const uint32_t sb = s_heads[h];
-      const uint32_t key = a.keys[sb];
-      const uint32_t se = h + 1 < nheads ? s_heads[h + 1] : SegmentEndSearch(a.keys, p1, end, key);
-      // A key or reference naming nothing of the push (a damaged workspace)
-      // is not used as an address: its loads read zero and the row is not
-      // written.  The reference checks see the same words in every lane.
-      const KeyParts kp = SplitKey(key, a.row_bits);
-      const TableDesc& T = s_t[min(kp.table, a.tables - 1)];
-      bool ok = KeyInRange(kp, a.tables, T.rows) && (!a.reduce || a.vals[sb] < a.n);
-      const uint64_t slot = ok ? kp.slot : 0;
-      const uint32_t dim = T.dim;
-      const uint64_t u = a.reduce && ok ? a.occ2u[a.vals[sb]] : 0;
-      auto ref_ok = [&](uint64_t w) {
-        const RefParts rp = SplitRef(w);
-        return RefInRange(rp, a.features, s_rows[min(rp.feature, a.features - 1)]);
-      };
+      const Row row = row_of(h);
+      if (row.se - row.sb > kBlockRowRefs) continue;
+      const TableDesc& T = sh.t[min(row.kp.table, a.tables - 1)];
+      bool ok = row.ok;
+      const uint32_t dim = T.dim, sb = row.sb, cnt = row.se - row.sb;
+      const SortedRefs refs{a.rs + sb, sh.grad, sh.rows, safe, a.features, dim};
       if (!kGeneric) {
         const uint32_t c = lig * 4;
         const bool active = c < dim;
+        const uint32_t cl = active ? c : 0;
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (uint32_t base = sb; base < se; base += G) {
-          const uint32_t cnt = min(G, se - base);
-          const uint64_t my = lig < cnt ? a.rs[base + lig] : 0ull;
-          for (uint32_t k = 0; k < cnt; k += 4) {
-            float4 x[4];
-            float s[4];
+        for (uint32_t k = 0; k < cnt; k += 4) {
+          float4 x[4];
+          float s[4];
+          uint64_t w[4];
 #pragma unroll
-            for (uint32_t q = 0; q < 4; ++q) {
-              const uint64_t w = __shfl(my, int(k + q), int(G));
-              const uint32_t ref = uint32_t(w);
-              s[q] = __uint_as_float(uint32_t(w >> 32));
-              const bool in = k + q < cnt && ref_ok(w);
-              if (k + q < cnt && !in) ok = false;
-              const float* src = s_grad[ref >> kRefRowBits] +
-                                 uint64_t(ref & ((1u << kRefRowBits) - 1)) * dim + c;
-              x[q] = (in && active) ? Load4(src) : make_float4(0.f, 0.f, 0.f, 0.f);
-            }
+          for (uint32_t q = 0; q < 4; ++q) w[q] = refs.Load(min(k + q, cnt - 1));
 #pragma unroll
-            for (uint32_t q = 0; q < 4; ++q)
-              if (k + q < cnt) Accumulate4(acc, x[q], s[q]);
-          }
+          for (uint32_t q = 0; q < 4; ++q) x[q] = Load4(refs.Source(w[q], cl, s[q], ok));
+#pragma unroll
+          for (uint32_t q = 0; q < 4; ++q)
+            if (k + q < cnt) Accumulate4(acc, x[q], s[q]);
         }
         if (!ok) st.err |= EPS_HIP_STATUS_BAD_INDEX;
         if (!active || !ok) continue;
-        if (a.reduce) {
+        if (kReduce) {
           if (!(Finite(acc.x) && Finite(acc.y) && Finite(acc.z) && Finite(acc.w)))
             st.err |= EPS_HIP_STATUS_REDUCE_OVERFLOW;
-          Store4(a.reduce_out + u * a.reduce_stride + c, acc);
+          Store4(a.reduce_out + row.u * a.reduce_stride + c, acc);
         } else {
-          AdamRow4(T, slot, c, acc, write, st);
+          AdamRow4(T, row.kp.slot, c, acc, write, st);
         }
       } else {
         for (uint32_t c0 = 0; c0 < dim; c0 += kWave) {
           const uint32_t c = c0 + lig;
           const bool active = c < dim;
+          const uint32_t cl = active ? c : c0;
           float acc = 0.f;
-          for (uint32_t base = sb; base < se; base += kWave) {
-            const uint32_t cnt = min(kWave, se - base);
-            const uint64_t my = lig < cnt ? a.rs[base + lig] : 0ull;
-            for (uint32_t k = 0; k < cnt; ++k) {
-              const uint64_t w = __shfl(my, int(k), int(kWave));
-              const uint32_t ref = uint32_t(w);
-              const float s = __uint_as_float(uint32_t(w >> 32));
-              const bool in = ref_ok(w);
-              if (!in) ok = false;
-              const float* src = s_grad[ref >> kRefRowBits] +
-                                 uint64_t(ref & ((1u << kRefRowBits) - 1)) * dim;
-              const float x = active && in ? LoadF(src + c) : 0.f;
-              acc = acc + x * s;
-            }
+          for (uint32_t k = 0; k < cnt; k += 8) {
+            float x[8], s[8];
+            uint64_t w[8];
+#pragma unroll
+            for (uint32_t q = 0; q < 8; ++q) w[q] = refs.Load(min(k + q, cnt - 1));
+#pragma unroll
+            for (uint32_t q = 0; q < 8; ++q) x[q] = LoadF(refs.Source(w[q], cl, s[q], ok));
+#pragma unroll
+            for (uint32_t q = 0; q < 8; ++q)
+              if (k + q < cnt) acc = acc + x[q] * s[q];
           }
           if (!ok) st.err |= EPS_HIP_STATUS_BAD_INDEX;
           if (!active || !ok) continue;
-          if (a.reduce) {
+          if (kReduce) {
             if (!Finite(acc)) st.err |= EPS_HIP_STATUS_REDUCE_OVERFLOW;
-            a.reduce_out[u * a.reduce_stride + c] = acc;
+            a.reduce_out[row.u * a.reduce_stride + c] = acc;
           } else {
-            AdamRow1(T, slot, c, acc, write, st);
+            AdamRow1(T, row.kp.slot, c, acc, write, st);
           }
+        }
+      }
+    }
+    // The window's long rows, one after another.
+    for (uint32_t h = 0; h < nheads; ++h) {
+      if ((h + 1 < nheads ? sh.heads[h + 1] : last_end) - sh.heads[h] <= kBlockRowRefs) continue;
+      const Row row = row_of(h);
+      const TableDesc& T = sh.t[min(row.kp.table, a.tables - 1)];
+      const SortedRefs refs{a.rs + row.sb, sh.grad, sh.rows, safe, a.features, T.dim};
+      for (uint32_t c0 = 0; c0 < T.dim; c0 += kBlock) {
+        bool ok = row.ok;
+        const float acc = BlockRowSum<!kGeneric>(sh.tile, refs, row.se - row.sb, T.dim, c0, 0.f, ok);
+        if (!ok) sh.bad = 1;
+        __syncthreads();
+        ok = sh.bad == 0;
+        __syncthreads();
+        if (threadIdx.x == 0) sh.bad = 0;
+        if (!ok) st.err |= EPS_HIP_STATUS_BAD_INDEX;
+        const uint32_t c = c0 + threadIdx.x;
+        if (c >= T.dim || !ok) continue;
+        if (kReduce) {
+          if (!Finite(acc)) st.err |= EPS_HIP_STATUS_REDUCE_OVERFLOW;
+          a.reduce_out[row.u * a.reduce_stride + c] = acc;
+        } else {
+          AdamRow1(T, row.kp.slot, c, acc, write, st);
         }
       }
     }
     __syncthreads();
   }
-  FinishBlock(st, ctrl, a.bounds, write && !a.reduce);
+}
+
+__device__ __forceinline__ void StageSorted(const FusedArgs& a, SortedShared& sh) {
+  CopyWords(sh.t, a.t, sizeof(a.t));
+  CopyWords(sh.grad, a.grad, sizeof(a.grad));
+  CopyWords(sh.rows, a.grad_rows, sizeof(a.grad_rows));
+}
+
+// Adam of the generic class (one wavefront per row, scalar columns), and the
+// checked apply of every class.
+__global__ void __launch_bounds__(kBlock) SortedUpdateKernel(FusedArgs a) {
+  // The checked apply nearly always has nothing to do.
+  if (a.role == kFallback && a.ctrl->mode != kChecked) return;
+  __shared__ SortedShared sh;
+  StageSorted(a, sh);
+  Control* ctrl = a.ctrl;
+  bool write = true;
+  if (!LaunchGate(ctrl, sh.t, a.gs, a.role, &sh.mode, write)) return;
+  // The classes' sorted positions, from the workspace, kept inside the push's.
+  const uint32_t first = ctrl->class_start[a.cls], last = ctrl->class_start[a.cls_end];
+  const uint32_t end = min(last, a.n), start = min(first, end);
+  RowStats st;
+  __syncthreads();
+  SortedRows<true, false>(a, sh, start, end, 6, PositionsPerBlock(kClasses - 1), blockIdx.x, gridDim.x, a.vblocks,
+                          write, st);
+  FinishBlock(st, ctrl, a.bounds, write);
+}
+
+// Reduced gradients of every class in one launch (class c has the blocks
+// [class_block[c], class_block[c + 1])): the classes' long rows then overlap.
+__global__ void __launch_bounds__(kBlock) SortedReduceKernel(FusedArgs a) {
+  __shared__ SortedShared sh;
+  StageSorted(a, sh);
+  Control* ctrl = a.ctrl;
+  uint32_t cls = 0;
+#pragma unroll
+  for (uint32_t c = 1; c < kClasses; ++c) cls += blockIdx.x >= a.class_block[c];
+  const uint32_t first = ctrl->class_start[cls], last = ctrl->class_start[cls + 1];
+  const uint32_t end = min(last, a.n), start = min(first, end);
+  const uint32_t block = blockIdx.x - a.class_block[cls];
+  RowStats st;
+  __syncthreads();
+  if (cls + 1 == kClasses)
+    SortedRows<true, true>(a, sh, start, end, 6, PositionsPerBlock(cls), block, block + 1, block + 1, false, st);
+  else
+    SortedRows<false, true>(a, sh, start, end, cls + 2, PositionsPerBlock(cls), block, block + 1, block + 1, false, st);
+  FinishBlock(st, ctrl, nullptr, false);
 }
 
 // ---------------------------------------------------------------------------
@@ -1407,30 +1608,97 @@ __global__ void __launch_bounds__(kBlock) RowUpdateKernel(RowArgs a) {
     if (!kGeneric) {
       const uint32_t c = lig * 4;
       const bool active = c < dim;
-      float4 g;
-      if (!a.offsets) {
-        g = active ? Load4(a.src + r * dim + c) : make_float4(0.f, 0.f, 0.f, 0.f);
-      } else {
-        g = make_float4(0.f, 0.f, 0.f, 0.f);
-        const uint64_t b = a.offsets[r], e = a.offsets[r + 1];
-        for (uint64_t j = b; j < e; ++j) {
-          const float s = a.scales[j];
-          const float4 x = active ? Load4(a.src + a.sources[j] * dim + c) : make_float4(0.f, 0.f, 0.f, 0.f);
-          Accumulate4(g, x, s);
-        }
-      }
+      const float4 g = active ? Load4(a.src + r * dim + c) : make_float4(0.f, 0.f, 0.f, 0.f);
       if (active) AdamRow4(T, slot, c, g, write, st);
     } else {
-      for (uint32_t c = lig; c < dim; c += kWave) {
-        float g;
-        if (!a.offsets) {
-          g = a.src[r * dim + c];
-        } else {
-          g = 0.f;
-          for (uint64_t j = a.offsets[r]; j < a.offsets[r + 1]; ++j)
-            g = g + a.src[a.sources[j] * dim + c] * a.scales[j];
+      for (uint32_t c = lig; c < dim; c += kWave) AdamRow1(T, slot, c, a.src[r * dim + c], write, st);
+    }
+  }
+  FinishBlock(st, ctrl, a.bounds, write);
+}
+
+constexpr uint64_t kCsrPiece = 1ull << 30;  // references of one BlockRowSum (it counts in 32 bits)
+
+// CSR rows.  Row r belongs to virtual block r % vblocks: a packet lists its
+// rows in first-occurrence order, so its long rows crowd at its start, and
+// neighbours go to different blocks.  A row of up to kBlockRowRefs references
+// takes one group, four gradient rows in flight; the block sums a longer one
+// (4,099 mean bags, 43,000 references of 11,900 rows of dim 64, the longest
+// row 3,900: one group a row, one reference in flight, 768 us; 85 us so).
+template <bool kGeneric>
+__global__ void __launch_bounds__(kBlock) CsrUpdateKernel(RowArgs a) {
+  __shared__ TableDesc s_t[1];
+  __shared__ uint32_t s_mode;
+  __shared__ __align__(16) float s_tile[kLongTile];
+  Control* ctrl = a.ctrl;
+  if (threadIdx.x == 0) s_t[0] = a.t;
+  bool write = false;
+  if (!LaunchGate(ctrl, s_t, a.gs, a.role, &s_mode, write)) return;
+  const TableDesc T = a.t;
+  const uint32_t dim = T.dim;
+  const uint32_t G = kGeneric ? kWave : (1u << a.log2g);
+  const uint32_t lig = threadIdx.x & (G - 1);
+  const uint32_t gid = threadIdx.x / G, ngroups = kBlock / G;
+  RowStats st;
+  for (uint32_t vb = blockIdx.x; vb < a.vblocks; vb += gridDim.x) {
+    const uint64_t r = uint64_t(gid) * a.vblocks + vb;
+    bool ok = true;  // the gradient scan has checked every source
+    if (r < a.rows) {
+      const uint64_t slot = a.slots[r], b = a.offsets[r], e = a.offsets[r + 1];
+      const uint32_t cnt = e > b ? uint32_t(min<uint64_t>(e - b, kBlockRowRefs + 1)) : 0u;
+      const CsrRefs refs{a.sources + b, a.scales + b, a.src, dim};
+      if (cnt > kBlockRowRefs) {
+        // below
+      } else if (!kGeneric) {
+        const uint32_t c = lig * 4;
+        const bool active = c < dim;
+        const uint32_t cl = active ? c : 0;
+        float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (uint32_t k = 0; k < cnt; k += 4) {
+          float4 x[4];
+          float s[4];
+          CsrRefs::Word w[4];
+#pragma unroll
+          for (uint32_t q = 0; q < 4; ++q) w[q] = refs.Load(min(k + q, cnt - 1));
+#pragma unroll
+          for (uint32_t q = 0; q < 4; ++q) x[q] = Load4(refs.Source(w[q], cl, s[q], ok));
+#pragma unroll
+          for (uint32_t q = 0; q < 4; ++q)
+            if (k + q < cnt) Accumulate4(g, x[q], s[q]);
         }
-        AdamRow1(T, slot, c, g, write, st);
+        if (active) AdamRow4(T, slot, c, g, write, st);
+      } else {
+        for (uint32_t c = lig; c < dim; c += kWave) {
+          float g = 0.f;
+          for (uint32_t k = 0; k < cnt; k += 8) {
+            float x[8], s[8];
+            CsrRefs::Word w[8];
+#pragma unroll
+            for (uint32_t q = 0; q < 8; ++q) w[q] = refs.Load(min(k + q, cnt - 1));
+#pragma unroll
+            for (uint32_t q = 0; q < 8; ++q) x[q] = LoadF(refs.Source(w[q], c, s[q], ok));
+#pragma unroll
+            for (uint32_t q = 0; q < 8; ++q)
+              if (k + q < cnt) g = g + x[q] * s[q];
+          }
+          AdamRow1(T, slot, c, g, write, st);
+        }
+      }
+    }
+    // The block's long rows, one after another (uniform over the block).
+    for (uint32_t i = 0; i < ngroups; ++i) {
+      const uint64_t row = uint64_t(i) * a.vblocks + vb;
+      if (row >= a.rows) break;
+      const uint64_t b = a.offsets[row], e = a.offsets[row + 1];
+      if (e <= b || e - b <= kBlockRowRefs) continue;
+      const uint64_t slot = a.slots[row];
+      for (uint32_t c0 = 0; c0 < dim; c0 += kBlock) {
+        float g = 0.f;
+        for (uint64_t at = b; at < e; at += kCsrPiece)
+          g = BlockRowSum<!kGeneric>(s_tile, CsrRefs{a.sources + at, a.scales + at, a.src, dim},
+                                     uint32_t(min(e - at, kCsrPiece)), dim, c0, g, ok);
+        const uint32_t c = c0 + threadIdx.x;
+        if (c < dim) AdamRow1(T, slot, c, g, write, st);
       }
     }
   }
@@ -1617,7 +1885,6 @@ int RunSorted(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, 
   a.ctrl = reinterpret_cast<Control*>(ws);
   a.bounds = bounds;
   a.row_bits = plan.row_bits;
-  a.reduce = reduce ? 1 : 0;
   a.tables = table_count;
   a.features = feature_count;
   a.n = uint32_t(plan.occurrences);
@@ -1772,35 +2039,39 @@ int RunSorted(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, 
       if (overlap && !joined) EPS_HIP_TRY(Check(hipEventRecord(ov->join, ov->side), "update join"));
     }
   }
-  for (uint32_t cls = 0; cls < kClasses; ++cls) {
-    if (!plan.class_occurrences[cls]) continue;
-    if (!reduce && cls + 1 < kClasses) continue;  // handled above
-    a.cls = cls;
-    a.cls_end = cls + 1;
-    a.log2g = cls + 2;
-    a.ppb = PositionsPerBlock(cls);
-    const uint64_t vb = (plan.class_occurrences[cls] + a.ppb - 1) / a.ppb;
-    a.vblocks = uint32_t(vb);
-    auto kernel = cls == 5 ? SortedUpdateKernel<true> : SortedUpdateKernel<false>;
-    if (phases & kPrimary) {
-      a.role = role;
-      role = kFollow;
-      hipLaunchKernelGGL(kernel, dim3(a.vblocks), dim3(kBlock), 0, s, a);
-      EPS_HIP_LAUNCHED("sorted update");
+  if (reduce) {
+    uint64_t blocks = 0;
+    for (uint32_t cls = 0; cls < kClasses; ++cls) {
+      a.class_block[cls] = uint32_t(blocks);
+      blocks += (plan.class_occurrences[cls] + PositionsPerBlock(cls) - 1) / PositionsPerBlock(cls);
     }
+    a.class_block[kClasses] = uint32_t(blocks);
+    hipLaunchKernelGGL(SortedReduceKernel, dim3(unsigned(blocks)), dim3(kBlock), 0, s, a);
+    EPS_HIP_LAUNCHED("sorted reduce");
+    return EPS_HIP_OK;
+  }
+  // The generic class.
+  if ((phases & kPrimary) && plan.class_occurrences[kClasses - 1]) {
+    const uint32_t ppb = PositionsPerBlock(kClasses - 1);
+    a.cls = kClasses - 1;
+    a.cls_end = kClasses;
+    a.vblocks = uint32_t((plan.class_occurrences[kClasses - 1] + ppb - 1) / ppb);
+    a.role = role;
+    hipLaunchKernelGGL(SortedUpdateKernel, dim3(a.vblocks), dim3(kBlock), 0, s, a);
+    EPS_HIP_LAUNCHED("sorted update");
   }
   if (overlap && (phases & kPrimary)) EPS_HIP_TRY(Check(hipStreamWaitEvent(s, ov->join, 0), "hot-row join wait"));
   // The checked apply (after a validate-only pass) is one launch over every
   // class, one wavefront per row: it usually exits at once, and when it runs
   // it adds each row's references in the same order as the passes above.
-  if (!reduce && (phases & kSecond)) {
+  if (phases & kSecond) {
+    const uint32_t ppb = PositionsPerBlock(kClasses - 1);
     a.cls = 0;
     a.cls_end = kClasses;
-    a.ppb = PositionsPerBlock(kClasses - 1);
-    a.vblocks = uint32_t((plan.occurrences + a.ppb - 1) / a.ppb);
+    a.vblocks = uint32_t((plan.occurrences + ppb - 1) / ppb);
     a.role = kFallback;
     if (a.vblocks) {
-      hipLaunchKernelGGL(SortedUpdateKernel<true>, dim3(std::min<uint32_t>(a.vblocks, kSecondGrid)),
+      hipLaunchKernelGGL(SortedUpdateKernel, dim3(std::min<uint32_t>(a.vblocks, kSecondGrid)),
                          dim3(kBlock), 0, s, a);
       EPS_HIP_LAUNCHED("sorted update (checked apply)");
     }
@@ -2003,7 +2274,8 @@ static int RunRows(const eps_hip_table* table, const eps_hip_optimizer* optimize
   const uint64_t vb = (rows + groups - 1) / groups;
   if (vb > 0xffffffffull) return Fail(EPS_HIP_CAPACITY_EXCEEDED, "too many rows");
   a.vblocks = uint32_t(vb);
-  auto kernel = generic ? RowUpdateKernel<true> : RowUpdateKernel<false>;
+  auto kernel = offsets ? (generic ? CsrUpdateKernel<true> : CsrUpdateKernel<false>)
+                        : (generic ? RowUpdateKernel<true> : RowUpdateKernel<false>);
   a.role = kDecide;
   hipLaunchKernelGGL(kernel, dim3(a.vblocks), dim3(kBlock), 0, s, a);
   EPS_HIP_LAUNCHED("row update");

@@ -15,9 +15,9 @@ inline uint32_t DimClass(uint32_t dim) {
   return log2g - 2;
 }
 
-// Positions of the sorted reference array handled by one block of the fused
-// update, per class: two segments' worth per sub-wavefront group.
-inline uint32_t PositionsPerBlock(uint32_t cls) {
+// Positions of the sorted reference array handled by one block of the sorted
+// driver, per class: two segments' worth per sub-wavefront group.
+EPS_HD uint32_t PositionsPerBlock(uint32_t cls) {
   return cls == 5 ? 8u : 2u * (kBlock >> (cls + 2));
 }
 

@@ -1,0 +1,101 @@
+"""Rows summed by a whole block (more than 32 references) beside rows summed by
+one lane group, at the edges of both: the reduce entry point, a push of the
+generic dimension class and CSR packets, bit-exact against the oracle (sums are
+taken in reference order from +0, so the tolerance is 0 ULP)."""
+import numpy as np
+import pytest
+
+import oracle
+from parity import assert_close, oracle_store
+from test_gpu_push import check_unique_reduce
+
+pytestmark = pytest.mark.gpu
+F32 = np.float32
+
+
+def lengths_of(dim):
+    """Row lengths around the hand-over to the block and its tiles."""
+    vector = dim % 4 == 0 and dim <= 256
+    width = dim // 4 if vector else min(dim, 256)
+    lanes = 4
+    while lanes < width:
+        lanes *= 2
+    tile = (8 if vector else 16) * (256 // lanes)
+    return [1, 2, 4, 5, 8, 9, 31, 32, 33, 48, 49] + [max(tile + k, 33) for k in (-1, 0, 1)] + \
+        [max(2 * tile, 33), 2 * tile + 7, 3 * tile + 1]
+
+
+def feature_of(W, rng, dim, lengths, rows):
+    slots = rng.permutation(rows)[: len(lengths)].astype(np.uint64)
+    keys = rng.permutation(np.repeat(slots, lengths))
+    bags = len(keys) // 3 + 1
+    cuts = np.sort(rng.integers(0, len(keys) + 1, bags - 1))
+    offsets = np.concatenate([[0], cuts, [len(keys)]]).astype(np.uint64)
+    weights = rng.normal(0, 1, len(keys)).astype(F32)
+    grad = rng.normal(0, 1e-2, (bags, dim)).astype(F32)
+    return W.Feature(0, 0, W.WEIGHTED_SUM, keys, offsets, np.diff(offsets), weights, grad)
+
+
+@pytest.mark.parametrize("dim", [4, 12, 64, 100, 128, 256, 3, 10, 50, 257, 300, 520])
+def test_reduce_long_rows(torch_gpu, pkg, dim):
+    torch, W, H = torch_gpu, pkg.workloads, pkg.eps_hip
+    rng = np.random.default_rng(dim)
+    lengths = lengths_of(dim)
+    specs = [W.TableSpec(0, dim, 400, seed=3)]
+    feats = [feature_of(W, rng, dim, lengths, specs[0].rows)]
+    print(f"case: dim={dim} row lengths {lengths}", flush=True)
+    check_unique_reduce(torch, W, H, specs, feats)
+
+
+@pytest.mark.parametrize("dim", [3, 50, 300])
+def test_push_long_generic_rows(torch_gpu, pkg, dim):
+    torch, W, H = torch_gpu, pkg.workloads, pkg.eps_hip
+    rng = np.random.default_rng(1000 + dim)
+    spec = W.TableSpec(0, dim, 400, seed=4)
+    f = feature_of(W, rng, dim, lengths_of(dim), spec.rows)
+    print(f"case: dim={dim} occurrences={len(f.keys)}", flush=True)
+    shard = H.DeviceShard(torch, [spec])
+    shard.init_rows()
+    dev = [H.DeviceFeature(torch, f)]
+    shard.prepare(dev)
+    assert shard.push(dev) & H.STATUS_ERRORS == 0
+    store = oracle_store(spec)
+    store.prepare(f)
+    assert oracle.push([store], [f], [0], [f.gradient]) == 0
+    keys = store.keys()
+    want, _ = store.read_many(keys)
+    got = shard.read_rows(0, torch.from_numpy(keys.view(np.int64)).cuda()).cpu().numpy()
+    assert_close(got.reshape(want.shape), want, f"generic push dim={dim}", strict_ulp=0)
+
+
+@pytest.mark.parametrize("dim", [4, 64, 100, 256, 3, 50, 300])
+def test_compact_long_rows(torch_gpu, pkg, dim):
+    torch, W, H = torch_gpu, pkg.workloads, pkg.eps_hip
+    rng = np.random.default_rng(2000 + dim)
+    spec = W.TableSpec(0, dim, 4000, seed=5)
+    # An empty row, the edges, and enough short rows for several virtual blocks.
+    lengths = np.array([0] + lengths_of(dim) + list(rng.integers(0, 7, 700)))
+    rows, count = len(lengths), 300
+    slots = rng.permutation(spec.rows)[:rows]
+    offsets = np.concatenate([[0], np.cumsum(lengths)]).astype(np.uint64)
+    sources = rng.integers(0, count, int(offsets[-1])).astype(np.uint64)
+    scales = rng.random(len(sources)).astype(F32)
+    values = rng.normal(0, 1e-2, (count, dim)).astype(F32)
+    print(f"case: dim={dim} rows={rows} references={len(sources)}", flush=True)
+    shard = H.DeviceShard(torch, [spec])
+    shard.init_rows()
+    at = torch.from_numpy(slots).cuda()
+    before = shard.read_rows(0, at).cpu().numpy().reshape(rows, 3, dim)
+    cuda = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    status = shard.adam_compact(0, at, cuda(offsets.view(np.int64)), cuda(sources.view(np.int64)), cuda(scales),
+                                cuda(values))
+    assert status & H.STATUS_ERRORS == 0, f"{status:#x}"
+    g = np.zeros((rows, dim), F32)
+    for r in range(rows):
+        for j in range(int(offsets[r]), int(offsets[r + 1])):
+            g[r] = g[r] + values[sources[j]] * scales[j]
+    rc, w, m, v = oracle.adam_rows_ctx(before[:, 0], before[:, 1], before[:, 2], g, spec.beta1, spec.beta2, spec.eps,
+                                       spec.lr, spec.b1p, spec.b2p)
+    assert rc == 0
+    got = shard.read_rows(0, at).cpu().numpy().reshape(rows, 3, dim)
+    assert_close(got, np.stack([w, m, v], 1), f"compact dim={dim}", strict_ulp=0)
