@@ -16,22 +16,22 @@ constexpr uint32_t kBlock = 256;          // 4 wavefronts of 64
 constexpr uint32_t kWave = 64;
 constexpr uint64_t kHole = ~0ull;         // "row not on this device" (UINT64_MAX)
 constexpr uint32_t kBoundSlots = 64;      // spread of the bound atomics
-constexpr uint32_t kSortTile = 4096;      // keys per radix-sort tile (256 x 16)
-constexpr uint32_t kSortItems = 16;
-constexpr uint32_t kGroupTiles = 16;     // radix tiles per look-back group
+constexpr uint32_t kSortBlock = 1024;     // threads of a sort block
+constexpr uint32_t kSortTile = 4096;      // occurrences per sort tile
+constexpr uint32_t kSortItems = kSortTile / kSortBlock;
+constexpr uint32_t kGroupTiles = 16;      // radix tiles per look-back group
 constexpr uint32_t kMaxPasses = 4;
-constexpr uint32_t kRadixBits = 9;        // largest radix digit
+constexpr uint32_t kRadixBits = 10;       // largest radix digit
 constexpr uint32_t kDigits = 1u << kRadixBits;
-constexpr uint32_t kDigitsPerThread = kDigits / kBlock;  // the sort kernels assume two
-static_assert(kDigitsPerThread == 2, "radix digits per thread");
-constexpr uint32_t kKeygenItems = 8;      // occurrences per keygen thread
+// Digits of all passes of a sort at most: ceil(bits / 10) passes of equal
+// width sort 30 bits in three passes of 1,024 digits, 32 in four of 256.
+constexpr uint32_t kAllDigits = 3 * kDigits;
 constexpr uint32_t kClasses = 6;          // 5 vector widths + generic
 constexpr uint32_t kRefRowBits = 27;      // gradient row bits in a reference word
 static_assert(kRefRowBits == kGuardRefRowBits, "one reference word layout");
 constexpr uint32_t kLongRefs = 128;       // rows with more references take the sliced path
 
 constexpr uint32_t kSrcSlots = 64;        // spread of the gradient/scale maximum atomics
-constexpr uint32_t kHistCopies = 16;      // spread of the keygen histogram atomics
 constexpr uint32_t kXcds = 8;             // XCDs of an MI355X
 constexpr uint32_t kHotBuckets = 8;       // hot-row lists per XCD, by length (longest first)
 
@@ -88,23 +88,30 @@ struct Bounds { uint32_t v[kBoundSlots][4]; };
 // A hot row: its sorted positions [start, end) and its key.
 struct HotEntry { uint32_t start, end, key, pad; };
 
-// Workspace layout of a push, for `n` occurrences.
+// What a sort tile's key generation found: occurrences on this device, max
+// |scale| above 1.0 (float bits) and prepare-status bits.
+struct TileInfo { uint32_t valid, scale, status, pad; };
+
+// Workspace layout of a push, for `n` occurrences.  Tiles cover one feature
+// (key generation, first pass) or one table (later passes), so a push of up
+// to 32 of them has at most `tiles` tiles and `groups` look-back groups.
 struct PushLayout {
   uint64_t n, tiles, groups;
-  uint64_t hist, look, group_look, keys_a, keys_b, vals_a, vals_b, refscale, sorted_rs, flags,
+  uint64_t info, counts, hist, look, keys_a, keys_b, vals_a, vals_b, refscale, sorted_rs, flags,
       ranks, block_sums, long_list, total;
   // Capacity of each hot-row list (any one may hold every hot row).
   constexpr uint64_t HotCapacity() const { return n / kLongRefs + 1; }
   constexpr explicit PushLayout(uint64_t occurrences)
-      : n(occurrences), tiles(0), groups(0), hist(0), look(0), group_look(0), keys_a(0), keys_b(0), vals_a(0),
+      : n(occurrences), tiles(0), groups(0), info(0), counts(0), hist(0), look(0), keys_a(0), keys_b(0), vals_a(0),
         vals_b(0), refscale(0), sorted_rs(0), flags(0), ranks(0), block_sums(0), long_list(0), total(0) {
-    tiles = (n + kSortTile - 1) / kSortTile;
-    groups = (tiles + kGroupTiles - 1) / kGroupTiles;
+    tiles = n / kSortTile + EPS_HIP_MAX_FEATURES;
+    groups = tiles / kGroupTiles + EPS_HIP_MAX_TABLES;
     auto align = [](uint64_t x) { return (x + 255) & ~uint64_t(255); };
     uint64_t at = sizeof(Control);
-    hist = at; at = align(at + kHistCopies * kMaxPasses * kDigits * 4);
-    look = at; at = align(at + kMaxPasses * tiles * kDigits * 4);
-    group_look = at; at = align(at + kMaxPasses * groups * kDigits * 4);
+    info = at; at = align(at + tiles * sizeof(TileInfo));
+    counts = at; at = align(at + kAllDigits * tiles * 2);
+    hist = at; at = align(at + EPS_HIP_MAX_TABLES * kAllDigits * 4);
+    look = at; at = align(at + kAllDigits * (tiles + groups) * 4);
     keys_a = at; at = align(at + n * 4);
     keys_b = at; at = align(at + n * 4);
     vals_a = at; at = align(at + n * 4);

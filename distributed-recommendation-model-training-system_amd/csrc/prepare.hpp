@@ -21,9 +21,19 @@ EPS_HD uint32_t PositionsPerBlock(uint32_t cls) {
   return cls == 5 ? 8u : 2u * (kBlock >> (cls + 2));
 }
 
+// Pushes of up to this many occurrences and staged bag offsets are prepared by
+// one block (SmallPrepareKernel).
+constexpr uint32_t kSmallOccurrences = kSortTile, kSmallOffsets = 8192;
+
 struct PushPlan {
   uint64_t occurrences = 0;           // total over features (holes included)
-  uint32_t row_bits = 0, key_bits = 0, passes = 0;
+  uint32_t row_bits = 0, key_bits = 0;
+  // The sorted keys and occurrence indices end in the second buffer of each
+  // pair after an odd number of passes.  A small push is sorted by one block
+  // straight into the second buffers (passes 1); its digit widths are
+  // small_bits, over the whole key.
+  bool small = false;
+  uint32_t passes = 0, small_passes = 0;
   std::array<uint32_t, kMaxPasses> shift{}, bits{};
   // Fixed-size, so planning a push allocates nothing.
   std::array<uint32_t, EPS_HIP_MAX_TABLES> key_index{};    // call table index -> key index (class order)

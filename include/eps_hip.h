@@ -270,7 +270,7 @@ int eps_hip_reduce(const eps_hip_table* tables, uint32_t table_count,
  * is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops).  Same as eps_hip_prepare + eps_hip_push on
  * the same arguments, with the push workspace in a static device array of this
- * library (about 12 MB per GPU, held from the library's load until the process
+ * library (about 15 MB per GPU, held from the library's load until the process
  * ends) instead of a caller's buffer; pushes of more than
  * EPS_HIP_STATIC_MAX_OCCURRENCES occurrences are refused with
  * EPS_HIP_CAPACITY_EXCEEDED before anything is enqueued.  `status` (device
