@@ -4,11 +4,13 @@
 // (bags, or positions for sequence pooling) of one feature.  It stages the
 // tile's bag offsets and row slots in LDS (one coalesced pass, unique->slot
 // remap and range checks done once per occurrence), then sub-wavefront groups
-// of G = dim/4 lanes (rounded up to a power of two, 4..64) each own one output
-// row: lane l holds columns [4l, 4l+4) and adds the bag's rows with 128-bit
-// loads, strictly in occurrence order from +0.0f, as the reference does
-// (GatherKernel, src/cuda/cache_backend.cu:81-94; PrepareFeature,
-// src/access/batch_access.cpp:41-50).  The mean divide of the client
+// of G lanes (dim / V rounded up to a power of two, 4..64) each own one output
+// row: lane l holds columns [V*l, V*l+V) (and those 64*V further on, for rows
+// wider than a wavefront) and adds the bag's rows with loads of V floats,
+// strictly in occurrence order from +0.0f, as the reference does (GatherKernel,
+// src/cuda/cache_backend.cu:81-94; PrepareFeature,
+// src/access/batch_access.cpp:41-50).  V is the widest of 4, 2 and 1 that the
+// dimension, the stride and the buffers' alignment allow.  The mean divide of the client
 // (src/client/distributed_client.cpp:227-232; NormalizeMean,
 // src/cuda/cache_backend.cu:134-139) is fused into the store.
 #include "common.hpp"
@@ -16,6 +18,7 @@
 #include <algorithm>
 #include <cfloat>
 #include <mutex>
+#include <type_traits>
 
 namespace eps_hip {
 
@@ -32,9 +35,10 @@ namespace {
 
 constexpr uint32_t kIdCap = 1024;     // occurrences staged in LDS per tile (LDS sets the occupancy)
 constexpr uint32_t kGatherBatch = 8;  // source rows in flight per lane group
-constexpr uint32_t kGenericLog2 = 0xff;
 constexpr int kBufferWord3 = 0x00020000;         // raw buffer resource, dword data (gfx9 family)
-constexpr uint32_t kBufferOutside = 0xFFFFFFF0u;  // an offset past every buffer range
+// An offset past every buffer range, also with the columns of a row of up to
+// kBufferDim floats added to it.
+constexpr uint32_t kBufferOutside = 0xFFFE0000u, kBufferDim = 16384;
 typedef int EpsI4 __attribute__((ext_vector_type(4)));
 
 struct GatherDesc {
@@ -46,11 +50,14 @@ struct GatherDesc {
   const float* weights;
   float* output;
   uint64_t stride, rows, source_rows, remap_count;
-  uint32_t dim, pooling, block_begin, log2g, rows_per_block;
+  uint32_t dim, pooling, block_begin;
+  uint16_t log2g, rows_per_block, width, reserved;  // width: floats of a load
+  uint32_t pieces_magic;  // sequence parts: 2^32 / (dim / width), rounded up
   // Bytes of the source when they fit a 32-bit buffer range (0: they do not):
   // the row loads then go through a buffer resource, and the slots of a batch
   // past the bag's end (or holes) take an offset outside the range, which
-  // returns zeros without a memory request.
+  // returns zeros without a memory request.  Rows read with the range's whole
+  // stride lie inside it, whatever the dimension.
   uint32_t buffer_bytes;
 };
 struct GatherArgs {
@@ -72,158 +79,267 @@ __device__ __forceinline__ uint64_t ResolveSlot(const GatherDesc& d, uint64_t i,
   return idx;
 }
 
-__global__ void __launch_bounds__(kBlock) GatherKernel(GatherArgs args) {
-  const GatherDesc d = args.part[PartOf(args.part, args.count)];
-
-  __shared__ uint64_t s_off[129];
-  __shared__ uint64_t s_slot[kIdCap];
-  __shared__ float s_weight[kIdCap];
-  __shared__ uint32_t s_bad;
-
-  const bool seq = d.pooling == EPS_HIP_POOL_SEQUENCE;
-  const bool weighted = d.pooling == EPS_HIP_POOL_WEIGHTED_SUM;
-  const uint64_t row0 = uint64_t(blockIdx.x - d.block_begin) * d.rows_per_block;
-  if (row0 >= d.rows) return;
-  const uint64_t row_end = min(row0 + d.rows_per_block, d.rows);
-  const uint32_t nrows = uint32_t(row_end - row0);
-  if (threadIdx.x == 0) s_bad = 0;
-  if (!seq)
-    for (uint32_t r = threadIdx.x; r <= nrows; r += kBlock) s_off[r] = d.offsets[row0 + r];
-  __syncthreads();
-  const uint64_t occ_begin = seq ? row0 : s_off[0];
-  // A part without indices has no occurrences (every bag empty): nothing is
-  // read, and offsets that claim occurrences are reported as bad indices.
-  const bool none = d.indices == nullptr;
-  if (none && !seq && s_off[nrows] != s_off[0] && threadIdx.x == 0) s_bad = 1;
-  const uint64_t occ_end = none ? occ_begin : (seq ? row_end : s_off[nrows]);
-  const bool staged = occ_end - occ_begin <= kIdCap;
-  bool bad = false;
-  if (staged) {
-    for (uint64_t i = occ_begin + threadIdx.x; i < occ_end; i += kBlock) {
-      s_slot[i - occ_begin] = ResolveSlot(d, i, bad);
-      if (weighted) s_weight[i - occ_begin] = d.weights[i];
-    }
+// V floats of a row: a load, and a load through the part's buffer resource.
+template <uint32_t V> struct Columns { float c[V]; };
+template <uint32_t V>
+__device__ __forceinline__ Columns<V> LoadColumns(const float* p) {
+  Columns<V> r;
+  if constexpr (V == 4) {
+    const float4 x = Load4(p);
+    r.c[0] = x.x; r.c[1] = x.y; r.c[2] = x.z; r.c[3] = x.w;
+  } else if constexpr (V == 2) {
+    typedef float F2 __attribute__((ext_vector_type(2)));
+    const F2 x = *(const EPS_GLOBAL F2*)(p);
+    r.c[0] = x.x; r.c[1] = x.y;
+  } else {
+    r.c[0] = LoadF(p);
   }
-  __syncthreads();
+  return r;
+}
+template <uint32_t V>
+__device__ __forceinline__ Columns<V> LoadColumns(__amdgpu_buffer_rsrc_t rsrc, uint32_t at) {
+  Columns<V> r;
+  if constexpr (V == 4) {
+    const EpsI4 q = __builtin_amdgcn_raw_buffer_load_b128(rsrc, at, 0, 0);
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) r.c[k] = __int_as_float(q[k]);
+  } else if constexpr (V == 2) {
+    const auto q = __builtin_amdgcn_raw_buffer_load_b64(rsrc, at, 0, 0);
+    r.c[0] = __int_as_float(int(q[0]));
+    r.c[1] = __int_as_float(int(q[1]));
+  } else {
+    r.c[0] = __int_as_float(int(__builtin_amdgcn_raw_buffer_load_b32(rsrc, at, 0, 0)));
+  }
+  return r;
+}
+template <uint32_t V>
+__device__ __forceinline__ void StoreColumns(float* p, const Columns<V>& r) {
+  if constexpr (V == 4) {
+    Store4(p, make_float4(r.c[0], r.c[1], r.c[2], r.c[3]));
+  } else if constexpr (V == 2) {
+    typedef float F2 __attribute__((ext_vector_type(2)));
+    *(EPS_GLOBAL F2*)(p) = F2{r.c[0], r.c[1]};
+  } else {
+    StoreF(p, r.c[0]);
+  }
+}
 
-  if (d.log2g != kGenericLog2) {
-    const uint32_t G = 1u << d.log2g;
-    const uint32_t lig = threadIdx.x & (G - 1);
-    const uint32_t ngroups = kBlock >> d.log2g;
-    const uint32_t c = lig * 4;
+// Where each staged occurrence's row starts: its byte offset in the part's
+// buffer range (kBufferOutside: a hole), or, for sources past such a range,
+// its 64-bit byte offset (kHole: a hole).
+struct GatherShared {
+  uint64_t off[kBlock / 4 + 1];
+  union {
+    uint32_t at32[kIdCap + kGatherBatch];
+    uint64_t at64[kIdCap];
+  };
+  float weight[kIdCap + kGatherBatch];
+  uint32_t bad;
+};
+
+// A value that is the same in every lane, in scalar registers.
+__device__ __forceinline__ uint64_t Uniform(uint64_t x) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(x)), hi = __builtin_amdgcn_readfirstlane(uint32_t(x >> 32));
+  return lo | (uint64_t(hi) << 32);
+}
+
+// Stages occurrences [first, first + n) of a part (n <= kIdCap): the remap and
+// the range check are done once per occurrence.
+__device__ __forceinline__ void StageOccurrences(const GatherDesc& d, GatherShared& sh, uint64_t first, uint32_t n,
+                                                 bool& bad) {
+  for (uint32_t k = threadIdx.x; k < n; k += kBlock) {
+    const uint64_t slot = ResolveSlot(d, first + k, bad);
+    if (d.buffer_bytes) sh.at32[k] = slot == kHole ? kBufferOutside : uint32_t(slot * d.stride * 4);
+    else sh.at64[k] = slot == kHole ? kHole : slot * d.stride * 4;
+    if (d.pooling == EPS_HIP_POOL_WEIGHTED_SUM) sh.weight[k] = d.weights[first + k];
+  }
+}
+
+// The output rows row0 .. row0 + nrows of a pooled part, a group of 2^log2g
+// lanes per row (at most one row a group) and V columns a lane.  The block's
+// occurrences [occ_begin, occ_end) are staged kIdCap at a time, usually once.
+// Each is staged as the offset of its row, so that a load costs a lane one LDS
+// read and an add instead of a 64-bit multiply per row and lane, which bound
+// the launch: 26 x 4,096 bags of 1-20 rows of dim 64, 46 -> 41 us; 4 x 262,144
+// bags of 32 rows of dim 128 (38 GB of state, past a buffer range), 1,775 ->
+// 1,071 us.
+template <uint32_t V, bool kWeighted, bool kBuffered>
+__device__ __forceinline__ void PoolRows(const GatherDesc& d, GatherShared& sh, uint64_t row0, uint32_t nrows,
+                                         uint64_t occ_begin, uint64_t occ_end, bool& bad) {
+  const uint32_t G = 1u << d.log2g;
+  const uint32_t lig = threadIdx.x & (G - 1);
+  const uint32_t r = threadIdx.x >> d.log2g;
+  const bool once = occ_end - occ_begin <= kIdCap;
+  // One step for rows of up to 64 * V columns.
+  for (uint32_t c0 = 0; c0 < d.dim; c0 += G * V) {
+    const uint32_t c = c0 + lig * V;
     const bool active = c < d.dim;
-    for (uint32_t r = threadIdx.x >> d.log2g; r < nrows; r += ngroups) {
-      const uint64_t beg = seq ? row0 + r : s_off[r];
-      const uint64_t end = none ? beg : (seq ? row0 + r + 1 : s_off[r + 1]);
-      float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (staged && d.source_rows) {
-        // Staged slots: every load of a batch is issued before any is added,
-        // with no branch around a load (a hole or a position past the bag
-        // reads row 0, column 0 and is dropped; row 0 exists).
-        const uint32_t cl = active ? c : 0;
+    Columns<V> acc;
+#pragma unroll
+    for (uint32_t k = 0; k < V; ++k) acc.c[k] = 0.f;
+    auto add = [&](const Columns<V>& x, float a) {
+#pragma unroll
+      for (uint32_t k = 0; k < V; ++k) {
+        if (kWeighted) acc.c[k] += x.c[k] * a;
+        else acc.c[k] += x.c[k];
+      }
+    };
+    for (uint64_t chunk = occ_begin; chunk < occ_end; chunk += kIdCap) {
+      const uint32_t n = uint32_t(min<uint64_t>(kIdCap, occ_end - chunk));
+      if (c0 == 0 || !once) {
+        if (c0 != 0 || chunk != occ_begin) __syncthreads();  // the chunk before has been added
+        StageOccurrences(d, sh, chunk, n, bad);
+        __syncthreads();
+      }
+      // The row's staged occurrences [first, e).
+      if (r >= nrows || !active) continue;
+      const uint64_t from = max(sh.off[r], chunk), to = min(sh.off[r + 1], chunk + n);
+      if (from >= to) continue;
+      const uint32_t first = uint32_t(from - chunk), e = uint32_t(to - chunk);
+      if constexpr (kBuffered) {
+        // Through the buffer range: occurrences past the bag and holes read
+        // zeros without a memory request, and adding them (weighted: zero
+        // times a weight of zero) changes no sum, since one that starts at
+        // +0.0f is never -0.0f.  The loads of a batch are issued before any
+        // is added.
         const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<float*>(d.source), (short)0, int(d.buffer_bytes), kBufferWord3);
-        for (uint64_t pos = beg; pos < end; pos += kGatherBatch) {
-          float4 v[kGatherBatch];
-          float a[kGatherBatch];
+        for (uint32_t pos = first; pos < e; pos += kGatherBatch) {
+          Columns<V> v[kGatherBatch];
+          uint32_t at[kGatherBatch];
+#pragma unroll
+          for (uint32_t u = 0; u < kGatherBatch; ++u) at[u] = sh.at32[pos + u];
+#pragma unroll
+          for (uint32_t u = 0; u < kGatherBatch; ++u) {
+            at[u] = pos + u < e ? at[u] : kBufferOutside;
+            v[u] = LoadColumns<V>(rsrc, at[u] + c * 4);
+          }
+#pragma unroll
+          for (uint32_t u = 0; u < kGatherBatch; ++u)
+            add(v[u], !kWeighted ? 1.f : at[u] != kBufferOutside ? sh.weight[pos + u] : 0.f);
+        }
+      } else if (d.source_rows) {  // (without rows every occurrence is a hole)
+        // No branch around a load: a hole or a position past the bag reads
+        // row 0 and is dropped.
+        const char* source = reinterpret_cast<const char*>(d.source + c);
+        for (uint32_t pos = first; pos < e; pos += kGatherBatch) {
+          Columns<V> v[kGatherBatch];
           bool ok[kGatherBatch];
 #pragma unroll
           for (uint32_t u = 0; u < kGatherBatch; ++u) {
-            const uint64_t i = pos + u;
-            const uint32_t at = uint32_t(min(i, end - 1) - occ_begin);
-            const uint64_t slot = s_slot[at];
-            ok[u] = i < end && slot != kHole;
-            a[u] = weighted ? s_weight[at] : 1.f;
-            if (d.buffer_bytes) {
-              const uint32_t boff = ok[u] && active ? uint32_t((slot * d.stride + c) * 4) : kBufferOutside;
-              const EpsI4 q = __builtin_amdgcn_raw_buffer_load_b128(rsrc, boff, 0, 0);
-              v[u] = make_float4(__int_as_float(q[0]), __int_as_float(q[1]), __int_as_float(q[2]),
-                                 __int_as_float(q[3]));
-            } else {
-              v[u] = Load4(d.source + (ok[u] ? slot : 0) * d.stride + cl);
-            }
+            const uint64_t at = sh.at64[min(pos + u, e - 1)];
+            ok[u] = pos + u < e && at != kHole;
+            v[u] = LoadColumns<V>(reinterpret_cast<const float*>(source + (ok[u] ? at : 0)));
           }
 #pragma unroll
-          for (uint32_t u = 0; u < kGatherBatch; ++u) {
-            if (!ok[u]) continue;
-            if (weighted) {
-              acc.x += v[u].x * a[u]; acc.y += v[u].y * a[u];
-              acc.z += v[u].z * a[u]; acc.w += v[u].w * a[u];
-            } else {
-              acc.x += v[u].x; acc.y += v[u].y; acc.z += v[u].z; acc.w += v[u].w;
-            }
-          }
-        }
-      } else {
-        for (uint64_t pos = beg; pos < end; pos += 4) {
-          float4 v[4];
-          float a[4];
-          bool ok[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const uint64_t i = pos + u;
-            uint64_t slot = kHole;
-            a[u] = 1.f;
-            if (i < end) {
-              if (staged) {
-                slot = s_slot[i - occ_begin];
-                if (weighted) a[u] = s_weight[i - occ_begin];
-              } else {
-                slot = ResolveSlot(d, i, bad);
-                if (weighted) a[u] = d.weights[i];
-              }
-            }
-            ok[u] = slot != kHole;
-            v[u] = (ok[u] && active) ? Load4(d.source + slot * d.stride + c)
-                                     : make_float4(0.f, 0.f, 0.f, 0.f);
-          }
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            if (!ok[u]) continue;
-            if (weighted) {
-              acc.x += v[u].x * a[u]; acc.y += v[u].y * a[u];
-              acc.z += v[u].z * a[u]; acc.w += v[u].w * a[u];
-            } else {
-              acc.x += v[u].x; acc.y += v[u].y; acc.z += v[u].z; acc.w += v[u].w;
-            }
-          }
+          for (uint32_t u = 0; u < kGatherBatch; ++u)
+            if (ok[u]) add(v[u], kWeighted ? sh.weight[pos + u] : 1.f);
         }
       }
-      if (d.pooling == EPS_HIP_POOL_MEAN && d.lengths) {
-        const uint64_t len = d.lengths[row0 + r];
-        if (len) {
-          const float f = (float)len;
-          acc.x = acc.x / f; acc.y = acc.y / f; acc.z = acc.z / f; acc.w = acc.w / f;
-        }
-      }
-      if (active) Store4(d.output + (row0 + r) * d.dim + c, acc);
     }
-  } else {
-    // Generic shapes (dim % 4 != 0 or dim > 256): one wavefront per row,
-    // scalar columns, same per-column operation order.
-    const uint32_t lane = threadIdx.x & (kWave - 1);
-    for (uint32_t r = threadIdx.x / kWave; r < nrows; r += kBlock / kWave) {
-      const uint64_t beg = seq ? row0 + r : s_off[r];
-      const uint64_t end = none ? beg : (seq ? row0 + r + 1 : s_off[r + 1]);
-      float div = 0.f;
-      if (d.pooling == EPS_HIP_POOL_MEAN && d.lengths) div = (float)d.lengths[row0 + r];
-      for (uint32_t c = lane; c < d.dim; c += kWave) {
-        float acc = 0.f;
-        for (uint64_t i = beg; i < end; ++i) {
-          const uint64_t slot = staged ? s_slot[i - occ_begin] : ResolveSlot(d, i, bad);
-          if (slot == kHole) continue;
-          const float x = d.source[slot * d.stride + c];
-          if (weighted) acc += x * (staged ? s_weight[i - occ_begin] : d.weights[i]);
-          else acc += x;
-        }
-        if (div != 0.f) acc = acc / div;
-        d.output[(row0 + r) * d.dim + c] = acc;
+    if (r >= nrows || !active) continue;
+    if (d.pooling == EPS_HIP_POOL_MEAN && d.lengths) {
+      const uint64_t len = d.lengths[row0 + r];
+      if (len) {
+        const float f = (float)len;
+#pragma unroll
+        for (uint32_t k = 0; k < V; ++k) acc.c[k] = acc.c[k] / f;
       }
+    }
+    StoreColumns<V>(d.output + (row0 + r) * d.dim + c, acc);
+  }
+}
+
+// The output rows row0 .. row0 + nrows of a sequence part, each a copy of one
+// source row (through +0.0f, as a sum of one; zeros for a hole).  The block's
+// rows are one run of pieces of V columns, kGatherBatch of them in flight a
+// thread: with a lane group per row a group had one load in flight and most
+// lanes of a row wider than a wavefront's columns were idle (five tables of
+// 20,011 bags of dims 16 to 300, one of them 130,000 sequence rows of dim 300:
+// the launch 127 us, now 55).
+template <uint32_t V>
+__device__ __forceinline__ void CopyRows(const GatherDesc& d, const GatherShared& sh, uint64_t row0, uint32_t nrows) {
+  const uint32_t per_row = d.dim / V, total = nrows * per_row;
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(d.source), (short)0, int(d.buffer_bytes), kBufferWord3);
+  float* out = d.output + row0 * d.dim;
+  for (uint32_t first = threadIdx.x; first < total; first += kBlock * kGatherBatch) {
+    Columns<V> v[kGatherBatch];
+    bool ok[kGatherBatch];
+#pragma unroll
+    for (uint32_t u = 0; u < kGatherBatch; ++u) {
+      const uint32_t e = min(first + u * kBlock, total - 1);
+      // e / per_row: exact for the at most 2^14 pieces of a block (or one row).
+      const uint32_t r = per_row == 1 ? e : nrows > 1 ? __umulhi(e, d.pieces_magic) : 0u;
+      const uint32_t col = (e - r * per_row) * V;
+      if (d.buffer_bytes) {
+        v[u] = LoadColumns<V>(rsrc, sh.at32[r] + col * 4);  // a hole reads zeros
+        ok[u] = true;
+      } else {
+        const uint64_t at = sh.at64[r];
+        ok[u] = at != kHole;
+#pragma unroll
+        for (uint32_t k = 0; k < V; ++k) v[u].c[k] = 0.f;
+        if (d.source_rows)  // else every row is a hole
+          v[u] = LoadColumns<V>(reinterpret_cast<const float*>(reinterpret_cast<const char*>(d.source) + (ok[u] ? at : 0)) +
+                                (ok[u] ? col : 0u));
+      }
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kGatherBatch; ++u) {
+      if (first + u * kBlock >= total) continue;
+#pragma unroll
+      for (uint32_t k = 0; k < V; ++k) v[u].c[k] = ok[u] ? 0.f + v[u].c[k] : 0.f;
+      StoreColumns<V>(out + uint64_t(first + u * kBlock) * V, v[u]);
     }
   }
-  if (bad) s_bad = 1;
+}
+
+__global__ void __launch_bounds__(kBlock) GatherKernel(GatherArgs args) {
+  const GatherDesc d = args.part[PartOf(args.part, args.count)];
+
+  __shared__ GatherShared sh;
+
+  const bool seq = d.pooling == EPS_HIP_POOL_SEQUENCE;
+  const uint64_t row0 = uint64_t(blockIdx.x - d.block_begin) * d.rows_per_block;
+  if (row0 >= d.rows) return;
+  const uint32_t nrows = uint32_t(min<uint64_t>(d.rows_per_block, d.rows - row0));
+  if (threadIdx.x == 0) sh.bad = 0;
+  bool bad = false;
+  if (seq) {
+    StageOccurrences(d, sh, row0, nrows, bad);
+    __syncthreads();
+    if (d.width == 4) CopyRows<4>(d, sh, row0, nrows);
+    else if (d.width == 2) CopyRows<2>(d, sh, row0, nrows);
+    else CopyRows<1>(d, sh, row0, nrows);
+  } else {
+    for (uint32_t r = threadIdx.x; r <= nrows; r += kBlock) sh.off[r] = d.offsets[row0 + r];
+    __syncthreads();
+    const uint64_t occ_begin = Uniform(sh.off[0]);
+    // A part without indices has no occurrences (every bag empty): nothing is
+    // read, and offsets that claim occurrences are reported as bad indices.
+    const bool none = d.indices == nullptr;
+    if (none && sh.off[nrows] != occ_begin && threadIdx.x == 0) sh.bad = 1;
+    const uint64_t occ_end = none ? occ_begin : Uniform(sh.off[nrows]);
+    auto pool = [&](auto v, auto weighted, auto through) {
+      PoolRows<decltype(v)::value, decltype(weighted)::value, decltype(through)::value>(d, sh, row0, nrows, occ_begin,
+                                                                                       occ_end, bad);
+    };
+    auto with_width = [&](auto weighted, auto through) {
+      if (d.width == 4) pool(std::integral_constant<uint32_t, 4>{}, weighted, through);
+      else if (d.width == 2) pool(std::integral_constant<uint32_t, 2>{}, weighted, through);
+      else pool(std::integral_constant<uint32_t, 1>{}, weighted, through);
+    };
+    auto with_weights = [&](auto through) {
+      if (d.pooling == EPS_HIP_POOL_WEIGHTED_SUM) with_width(std::true_type{}, through);
+      else with_width(std::false_type{}, through);
+    };
+    if (d.buffer_bytes) with_weights(std::true_type{});
+    else with_weights(std::false_type{});
+  }
+  if (bad) sh.bad = 1;
   __syncthreads();
-  if (threadIdx.x == 0 && s_bad && args.status) atomicOr(args.status, EPS_HIP_STATUS_BAD_INDEX);
+  if (threadIdx.x == 0 && sh.bad && args.status) atomicOr(args.status, EPS_HIP_STATUS_BAD_INDEX);
 }
 
 __global__ void AddContributionKernel(float* output, const float* source, const uint64_t* positions,
@@ -612,19 +728,25 @@ int eps_hip_gather(const eps_hip_gather_part* parts, uint32_t count, uint32_t* s
     d.stride = in.stride; d.rows = in.rows; d.source_rows = in.source_rows;
     d.remap_count = in.remap_count; d.dim = in.dim; d.pooling = in.pooling;
     const uint64_t source_bytes = in.source_rows * in.stride * 4;
-    d.buffer_bytes = source_bytes && source_bytes < kBufferOutside && in.source_rows < (1ull << 32)
+    d.buffer_bytes = source_bytes && source_bytes <= kBufferOutside && in.source_rows < (1ull << 32) &&
+                             in.stride <= kBufferOutside && in.dim <= kBufferDim
                          ? uint32_t(source_bytes) : 0u;
-    const bool vec = in.dim % 4 == 0 && in.dim <= 256 && in.stride % 4 == 0 &&
-                     reinterpret_cast<uintptr_t>(in.source) % 16 == 0 &&
-                     reinterpret_cast<uintptr_t>(in.output) % 16 == 0;
-    if (vec) {
-      uint32_t log2g = 2;
-      while ((1u << log2g) < in.dim / 4) ++log2g;
-      d.log2g = log2g;
-      d.rows_per_block = kBlock >> log2g;  // one bag per lane group
-    } else {
-      d.log2g = kGenericLog2;
-      d.rows_per_block = 8;
+    // The widest load that every row and the output allow.
+    auto fits = [&](uint32_t v) {
+      return in.dim % v == 0 && in.stride % v == 0 && reinterpret_cast<uintptr_t>(in.source) % (4 * v) == 0 &&
+             reinterpret_cast<uintptr_t>(in.output) % (4 * v) == 0;
+    };
+    const uint32_t width = fits(4) ? 4u : fits(2) ? 2u : 1u;
+    uint32_t log2g = 2;
+    while (log2g < 6 && (width << log2g) < in.dim) ++log2g;
+    d.width = uint16_t(width);
+    d.log2g = uint16_t(log2g);
+    d.rows_per_block = uint16_t(kBlock >> log2g);  // one bag per lane group
+    if (in.pooling == EPS_HIP_POOL_SEQUENCE) {
+      // A batch of pieces per thread, staged slots permitting.
+      const uint32_t per_row = in.dim / width;
+      d.rows_per_block = uint16_t(std::min(std::max(kBlock * kGatherBatch / per_row, 1u), kIdCap));
+      d.pieces_magic = uint32_t((uint64_t(1) << 32) / per_row + (per_row > 1));
     }
     d.block_begin = blocks;
     const uint64_t b = (in.rows + d.rows_per_block - 1) / d.rows_per_block;
