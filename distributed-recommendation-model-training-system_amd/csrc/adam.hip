@@ -33,6 +33,7 @@
 #include <atomic>
 #include <cfloat>
 #include <cmath>
+#include <type_traits>
 
 namespace eps_hip {
 
@@ -940,8 +941,228 @@ __device__ __forceinline__ void PostCounter(uint32_t* counter, uint32_t value) {
     __hip_atomic_store(counter, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+constexpr uint32_t kLongDepth = 2;  // own chunks of rows a producer of a long unit keeps in flight (even)
+
+// One unit on a block of its own: the kS columns from col0 of a row of very
+// many references.  There is no stream to walk, and a chunk is always 4,096
+// products, so the adding wave is held up once per 4,096 / kS references.
+// Each producer has a tile of its own ([reference][column], which it writes
+// with 16-byte stores as the rows arrive), two own chunks of rows in flight
+// and the reference words of a third; the adding wave reads a tile a part of
+// 64 references at a time into one register buffer while it adds the other.
+// What bounds it is the adding wave's instruction rate (about one per six
+// cycles, whatever their kind): an add and half an LDS read a reference.  4 x
+// 8.4 M references, the hottest rows 977,000: 7.4 ns a reference in 64-reference
+// chunks with the stream walked between them (hot-row kernel 7.1 ms), 5.7 so
+// (5.6 ms; with one chunk of rows in flight 10, 9.8 ms).
+template <uint32_t kS>
+struct LongShape {
+  static constexpr uint32_t kChunk = 4096 / kS;            // references of a chunk
+  static constexpr uint32_t kQuads = kS / 4;
+  static constexpr uint32_t kRefsPerLoad = kWave / kQuads;
+  static constexpr uint32_t kLoads = kChunk / kRefsPerLoad;  // row loads of a producer lane per chunk
+  static constexpr uint32_t kParts = kChunk / kWave;
+  static constexpr uint32_t kWords = kChunk / kWave;  // reference words of a producer lane per chunk
+  static_assert(kLoads == 16 && kParts % 2 == 0, "long unit shape");
+};
+template <uint32_t kS>
+struct LongShared {
+  __align__(16) float tile[kProducers][4096];
+  // A producer's decoded references: entry [sub][i] is what its row load i
+  // brings to the lanes of `sub`.
+  const float* src[kProducers][LongShape<kS>::kRefsPerLoad][LongShape<kS>::kLoads];
+  float scale[kProducers][LongShape<kS>::kRefsPerLoad][LongShape<kS>::kLoads];
+  uint32_t ready[kProducers], used[kProducers];
+};
+
+template <uint32_t kS>
+__device__ void LongUnit(const VecArgs& a, LongShared<kS>& sh, const TableDesc* s_t, const float* const* s_grad,
+                         const uint64_t* s_rows, uint32_t* s_bad, uint32_t start, uint32_t end, uint32_t key,
+                         uint32_t col0, bool write, RowStats& st) {
+  using Shape = LongShape<kS>;
+  constexpr uint32_t kChunk = Shape::kChunk;
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave)));
+  start = __builtin_amdgcn_readfirstlane(start);
+  end = __builtin_amdgcn_readfirstlane(end);
+  const KeyParts kp = SplitKey(__builtin_amdgcn_readfirstlane(key), a.row_bits);
+  const TableDesc& T = s_t[min(kp.table, a.tables - 1)];
+  const bool key_ok = KeyInRange(kp, a.tables, T.rows);
+  const uint32_t dim = T.dim;
+  const uint32_t chunks = (end - start + kChunk - 1) / kChunk;
+  const float* idle = reinterpret_cast<const float*>(a.rs);
+  bool stalled = false;
+  if (wave == 0) {
+    __builtin_amdgcn_s_setprio(2);
+    const uint32_t c = lane % kS;
+    const bool mine = lane < kS && col0 + c < dim;
+    float* row = T.state + uint64_t(key_ok ? kp.slot : 0u) * dim * 3 + (mine ? col0 + c : 0u);
+    float w = 0.f, m = 0.f, v = 0.f;
+    if (key_ok) { w = LoadF(row); m = LoadF(row + dim); v = LoadF(row + 2 * dim); }
+    float acc = 0.f;
+    float xa[kWave], xb[kWave];
+    // Part h of tile t: rows kStep apart lie 256 bytes apart, so that a pair of
+    // them is one LDS access; one address a residue (opaque to the compiler,
+    // which would pair neighbours and take an address for each eight rows).
+    constexpr uint32_t kStep = kWave / kS;
+    uint32_t at[kStep];
+#pragma unroll
+    for (uint32_t k = 0; k < kStep; ++k) {
+      at[k] = k * kS + c;
+      if constexpr (kStep > 1) asm volatile("" : "+v"(at[k]));
+    }
+    auto read = [&](uint32_t t, uint32_t h, uint32_t r) {
+      return (&sh.tile[0][0])[at[r % kStep] + t * 4096 + h * (kWave * kS) + r / kStep * kWave];
+    };
+    // Chunk j lies in tile j % kProducers, whose number is a constant of the
+    // unrolled loop.  uses = j / kProducers + 1.
+    auto add_chunk = [&](uint32_t t, uint32_t j, uint32_t uses) {
+      const uint32_t next = (t + 1) % kProducers, next_uses = t + 1 == kProducers ? uses + 1 : uses;
+      uint32_t peek = 0;
+#pragma unroll
+      for (uint32_t h = 0; h < Shape::kParts; ++h) {
+        float* cur = h % 2 ? xb : xa;
+        float* nxt = h % 2 ? xa : xb;
+        const bool last = h + 1 == Shape::kParts;
+        // The part to add has arrived before the next part's reads go out.
+        __builtin_amdgcn_s_waitcnt(kLgkmZero);
+        __builtin_amdgcn_sched_barrier(0);
+        if (last) {
+          if (j + 1 < chunks && uint32_t(__builtin_amdgcn_readfirstlane(int(peek))) < next_uses &&
+              !WaitCounter(&sh.ready[next], next_uses, 0, a.spin_limit)) {
+            stalled = true;
+            return;
+          }
+          // Every value of this tile is in registers: its producer may have it
+          // back.  (A part past the last chunk is read all the same, from a
+          // tile in LDS, and dropped.  The LDS accesses of one wavefront are
+          // performed in order: the fence only holds the compiler.)
+          if (lane == 0)
+            __hip_atomic_store(&sh.used[t], uses, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+        } else if (h + 2 == Shape::kParts) {
+          // The next chunk's readiness is read along with the last part.
+          peek = __hip_atomic_load(&sh.ready[next], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // The next part's reads go out among the adds, two rows a read.
+#pragma unroll
+        for (uint32_t r = 0; r < kWave; r += 2 * kStep) {
+#pragma unroll
+          for (uint32_t k = r; k < r + 2 * kStep; ++k) nxt[k] = last ? read(next, 0, k) : read(t, h + 1, k);
+#pragma unroll
+          for (uint32_t k = r; k < r + 2 * kStep; ++k) acc = acc + cur[k];
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        asm volatile("" : "+v"(acc));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    if (!WaitCounter(&sh.ready[0], 1, 0, a.spin_limit)) {
+      stalled = true;
+    } else {
+#pragma unroll
+      for (uint32_t r = 0; r < kWave; ++r) xa[r] = read(0, 0, r);
+    }
+    for (uint32_t j = 0, uses = 1; j < chunks && !stalled; j += kProducers, ++uses) {
+#pragma unroll
+      for (uint32_t t = 0; t < kProducers; ++t)
+        if (j + t < chunks && !stalled) add_chunk(t, j + t, uses);
+    }
+    if (!key_ok) *s_bad = 1;
+    if (mine && key_ok && !stalled) {
+      AdamElement(T, acc, w, m, v, st);
+      if (write && !*s_bad) {
+        StoreF(row, w); StoreF(row + dim, m); StoreF(row + 2 * dim, v);
+      }
+    }
+  } else {
+    const uint32_t p = wave - 1;
+    const uint32_t quad = lane % Shape::kQuads, sub = lane / Shape::kQuads;
+    // Lanes whose columns lie past the row's dimension read the slice's first.
+    const uint32_t at = col0 + 4 * quad < dim ? 4 * quad : 0u;
+    float4 x[kLongDepth][Shape::kLoads];
+    float scale[kLongDepth][Shape::kLoads];
+    uint64_t word[2][Shape::kWords];  // lane l: references l, l + 64, ... of a chunk
+    float* tile = sh.tile[p] + sub * kS + 4 * quad;
+    // Own chunk k is chunk p + kProducers * k; past the row's end its words are
+    // the row's last, its products -0.0f (the identity of addition).
+    auto first_of = [&](uint32_t k) { return start + (p + kProducers * k) * kChunk; };  // (positions stay below 2^30)
+    auto load_words = [&](uint32_t k, uint64_t (&w)[Shape::kWords]) {
+#pragma unroll
+      for (uint32_t i = 0; i < Shape::kWords; ++i) w[i] = a.rs[min(first_of(k) + kWave * i + lane, end - 1)];
+    };
+    auto decode = [&](const uint64_t (&w)[Shape::kWords]) {
+#pragma unroll
+      for (uint32_t i = 0; i < Shape::kWords; ++i) {
+        const uint32_t r = kWave * i + lane;
+        const RefParts rp = SplitRef(w[i]);
+        const uint32_t f = min(rp.feature, a.features - 1);
+        const bool ok = RefInRange(rp, a.features, s_rows[f]);
+        if (!ok) *s_bad = 1;
+        sh.src[p][r % Shape::kRefsPerLoad][r / Shape::kRefsPerLoad] =
+            ok ? s_grad[f] + uint64_t(rp.row) * dim + col0 : idle;
+        sh.scale[p][r % Shape::kRefsPerLoad][r / Shape::kRefsPerLoad] = __uint_as_float(uint32_t(w[i] >> 32));
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    };
+    auto load_rows = [&](float4 (&xr)[Shape::kLoads], float (&sr)[Shape::kLoads]) {
+#pragma unroll
+      for (uint32_t i = 0; i < Shape::kLoads; ++i) xr[i] = Load4(sh.src[p][sub][i] + at);
+#pragma unroll
+      for (uint32_t i = 0; i < Shape::kLoads; ++i) sr[i] = sh.scale[p][sub][i];
+    };
+    const uint32_t own = chunks > p ? (chunks - p + kProducers - 1) / kProducers : 0u;
+    if (own) {
+      // Loads return in issue order, so the words of own chunk k + D + 1 go out
+      // before the rows of own chunk k + D: decoding them waits for no row.
+      load_words(0, word[0]);
+#pragma unroll
+      for (uint32_t k = 0; k < kLongDepth; ++k) {
+        decode(word[k % 2]);
+        load_words(k + 1, word[(k + 1) % 2]);
+        load_rows(x[k], scale[k]);
+      }
+      auto stage = [&](uint32_t k, uint32_t slot, uint64_t (&w)[Shape::kWords], uint64_t (&next)[Shape::kWords]) {
+        float4(&xr)[Shape::kLoads] = x[slot];
+        float(&sr)[Shape::kLoads] = scale[slot];
+        if (!stalled && !WaitCounter(&sh.used[p], k, 1, a.spin_limit)) stalled = true;
+        if (stalled) return;
+        const uint32_t first = first_of(k);
+        if (first + kChunk <= end) {
+#pragma unroll
+          for (uint32_t i = 0; i < Shape::kLoads; ++i)
+            *reinterpret_cast<float4*>(tile + i * (Shape::kRefsPerLoad * kS)) =
+                make_float4(xr[i].x * sr[i], xr[i].y * sr[i], xr[i].z * sr[i], xr[i].w * sr[i]);
+        } else {
+#pragma unroll
+          for (uint32_t i = 0; i < Shape::kLoads; ++i) {
+            const bool in = first + Shape::kRefsPerLoad * i + sub < end;
+            *reinterpret_cast<float4*>(tile + i * (Shape::kRefsPerLoad * kS)) =
+                make_float4(in ? xr[i].x * sr[i] : -0.f, in ? xr[i].y * sr[i] : -0.f, in ? xr[i].z * sr[i] : -0.f,
+                            in ? xr[i].w * sr[i] : -0.f);
+          }
+        }
+        PostCounter(&sh.ready[p], k + 1);
+        decode(w);                               // own chunk k + D
+        load_words(k + kLongDepth + 1, next);
+        load_rows(xr, sr);                       // own chunk k + D
+      };
+      for (uint32_t k = 0; k < own && !stalled; k += kLongDepth) {
+#pragma unroll
+        for (uint32_t d = 0; d < kLongDepth; ++d)
+          if (k + d < own) stage(k + d, d, word[(d + kLongDepth) % 2], word[(d + kLongDepth + 1) % 2]);
+      }
+    }
+  }
+  if (stalled) st.err |= EPS_HIP_STATUS_STALLED;
+}
+
 template <uint32_t kSlice, uint32_t kChunk>
-__global__ void __launch_bounds__(kHotBlock) HotSliceKernel(VecArgs a) {
+__global__ void __launch_bounds__(kHotBlock) __attribute__((amdgpu_waves_per_eu(kSlice == 32 ? 2 : 1)))
+HotSliceKernel(VecArgs a) {
   using Shape = HotShape<kSlice, kChunk>;
   constexpr uint32_t kHotQuads = Shape::kQuads;
   constexpr uint32_t kHotRefsPerLoad = Shape::kRefsPerLoad;
@@ -952,7 +1173,11 @@ __global__ void __launch_bounds__(kHotBlock) HotSliceKernel(VecArgs a) {
   constexpr uint32_t kDepth = Shape::kDepth;
   __shared__ TableDesc s_t[EPS_HIP_MAX_TABLES];
   __shared__ const float* s_grad[EPS_HIP_MAX_FEATURES];
-  __shared__ __align__(16) float s_tile[kHotRing][kSlice * kPitch];
+  // Pushes with very long rows (narrow units) give the longest a block each.
+  constexpr bool kLong = kSlice < kWave;
+  struct Tiles { __align__(16) float tile[kHotRing][kSlice * kPitch]; };
+  __shared__ union { Tiles t; std::conditional_t<kLong, LongShared<kLong ? kSlice : 32>, uint32_t> lone; } s_tiles;
+  auto& s_tile = s_tiles.t.tile;
   __shared__ float s_wmv[kHotRing][3][kSlice];
   __shared__ __align__(16) HotRefs<kSlice, kChunk> s_ref[kProducers];
   // ready[t]: chunks staged in tile t so far; used[t]: chunks added from it.
@@ -1021,6 +1246,21 @@ __global__ void __launch_bounds__(kHotBlock) HotSliceKernel(VecArgs a) {
     col0 = (local & slice_mask) * kSlice;
     return uint64_t(xcd * kHotBuckets + b) * a.hot_capacity + (local >> a.slice_bits);
   };
+  if constexpr (kLong) {
+    if (me < own) {
+      uint32_t col0;
+      HotEntry e = a.hot[entry_of(me, col0)];
+      if (!sane(e.start, e.end)) s_bad = 1;
+      if (threadIdx.x < kProducers) s_tiles.lone.ready[threadIdx.x] = s_tiles.lone.used[threadIdx.x] = 0;
+      __syncthreads();
+      if (col0 < s_t[min(e.key >> a.row_bits, a.tables - 1)].dim)
+        LongUnit<kSlice>(a, s_tiles.lone, s_t, s_grad, s_rows, &s_bad, e.start, e.end, e.key, col0, write, st);
+      __syncthreads();
+      if (s_bad) st.err |= EPS_HIP_STATUS_BAD_INDEX;
+      FinishBlock<kHotBlock / kWave>(st, ctrl, a.bounds, write);
+      return;
+    }
+  }
   // The headers of the block's first kUnitCache units are staged in LDS once,
   // so walking the stream costs each wave an LDS read per unit.  (A scalar
   // load per unit would stall every wave's next LDS wait until it returns:
