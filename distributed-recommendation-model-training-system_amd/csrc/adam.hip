@@ -1983,11 +1983,26 @@ uint32_t Log2G(uint32_t dim) {
   return log2g;
 }
 
+// A launch that also records `done` when the kernel completes (nullptr: a
+// plain launch).  The event then rides on the kernel's own completion signal,
+// with no marker packet after it in the stream.  For the join of the side
+// stream: 26 tables of ~43,000 references, 0.2723 -> 0.2687 ms a step over six
+// paired runs on one box (each faster than its pair), 0.2708 -> 0.2701 over
+// four on another; 65,536 pairs on one table 0.111 -> 0.109 ms.
+template <typename... Args>
+void LaunchRecording(void (*kernel)(Args...), dim3 grid, dim3 block, hipStream_t s, hipEvent_t done,
+                     Args... args) {
+  if (done)
+    hipExtLaunchKernelGGL(kernel, grid, block, 0, s, nullptr, done, 0, args...);
+  else
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, args...);
+}
+
 // The gradient scan.  It always runs (one block at least), since its block 0
 // takes the bounds snapshot the guard decides from; the decision itself is
 // made by the first kernel of the update (DecideBlock).
-int LaunchGuard(const GuardArgs& g, uint64_t blocks, hipStream_t s) {
-  hipLaunchKernelGGL(GradMaxKernel, dim3(unsigned(std::max<uint64_t>(blocks, 1))), dim3(kBlock), 0, s, g);
+int LaunchGuard(const GuardArgs& g, uint64_t blocks, hipStream_t s, hipEvent_t done = nullptr) {
+  LaunchRecording(GradMaxKernel, dim3(unsigned(std::max<uint64_t>(blocks, 1))), dim3(kBlock), s, done, g);
   EPS_HIP_LAUNCHED("gradient guard");
   return EPS_HIP_OK;
 }
@@ -2053,7 +2068,8 @@ thread_local bool t_hot_row_overlap = true;
 // and kOneStream: every kernel on the caller's stream, the hot-row kernel
 // before the row kernels (no side stream or event is created or used, so the
 // push can be captured in a graph).
-constexpr int kPrimary = 1, kSecond = 2, kOneStream = 4;
+// kForked: the gradient scan has recorded the thread's fork event.
+constexpr int kPrimary = 1, kSecond = 2, kOneStream = 4, kForked = 8;
 constexpr uint64_t kVectorGrid = 4096;  // persistent grid cap of the vector kernels
 constexpr uint64_t kSecondGrid = 32;      // grid cap of the checked apply: it usually exits at
                                           // once, and a small grid launches faster
@@ -2063,21 +2079,6 @@ constexpr uint64_t kHotGrid = 512;      // two blocks per CU (LDS: four 17 KiB t
 // them most of the GPU (26 tables of ~43,000 references: 64 blocks 259 us a
 // step of pull + push, 256 blocks 236, 512 blocks 240).
 constexpr uint64_t kWideHotGrid = 256;
-
-// A launch that also records `done` when the kernel completes (nullptr: a
-// plain launch).  The event then rides on the kernel's own completion signal,
-// with no marker packet after it in the stream.  For the join of the side
-// stream: 26 tables of ~43,000 references, 0.2723 -> 0.2687 ms a step over six
-// paired runs on one box (each faster than its pair), 0.2708 -> 0.2701 over
-// four on another; 65,536 pairs on one table 0.111 -> 0.109 ms.
-template <typename... Args>
-void LaunchRecording(void (*kernel)(Args...), dim3 grid, dim3 block, hipStream_t s, hipEvent_t done,
-                     Args... args) {
-  if (done)
-    hipExtLaunchKernelGGL(kernel, grid, block, 0, s, nullptr, done, 0, args...);
-  else
-    hipLaunchKernelGGL(kernel, grid, block, 0, s, args...);
-}
 
 template <uint32_t kLog2G>
 int LaunchRowRun(unsigned grid, const VecArgs& a, hipStream_t s, hipEvent_t done) {
@@ -2108,6 +2109,20 @@ int LaunchVectorUpdate(uint32_t cls, uint32_t hot_slice, unsigned grid, const Ve
     case 4: return LaunchRowRun<6>(grid, a, s, done);
     default: return Fail(EPS_HIP_INVALID_ARGUMENT, "no vector kernel for this dimension class");
   }
+}
+
+// Bound on the hot rows of a push: a hot row takes more than kLongRefs
+// references of its own table, so no table adds more hot rows than its
+// references allow; a push with no such table (a few hundred pairs) launches no
+// hot-row kernel and no events.  `table_refs`: references per table.
+uint64_t HotRowBound(const eps_hip_table* tables, uint32_t table_count, const eps_hip_push_feature* features,
+                     uint32_t feature_count, uint64_t* table_refs) {
+  std::fill(table_refs, table_refs + EPS_HIP_MAX_TABLES, 0);
+  for (uint32_t f = 0; f < feature_count; ++f) table_refs[features[f].table] += features[f].occurrences;
+  uint64_t rows = 0;
+  for (uint32_t t = 0; t < table_count; ++t)
+    if (DimClass(tables[t].dim) < kClasses - 1) rows += table_refs[t] / (kLongRefs + 1);
+  return rows;
 }
 
 int RunSorted(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, uint32_t table_count,
@@ -2164,8 +2179,8 @@ int RunSorted(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, 
     va.gs = a.gs;
     va.spin_limit = SpinLimit();
     va.row_bits = plan.row_bits;
-    uint64_t table_refs[EPS_HIP_MAX_TABLES] = {};
-    for (uint32_t f = 0; f < feature_count; ++f) table_refs[features[f].table] += features[f].occurrences;
+    uint64_t table_refs[EPS_HIP_MAX_TABLES];
+    const uint64_t hot_rows = HotRowBound(tables, table_count, features, feature_count, table_refs);
     const bool long_rows = *std::max_element(table_refs, table_refs + table_count) >= kOverlapTableRefs;
     uint64_t vector_occurrences = 0;
     for (uint32_t cls = 0; cls + 1 < kClasses; ++cls) vector_occurrences += plan.class_occurrences[cls];
@@ -2193,12 +2208,6 @@ int RunSorted(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, 
         slices = std::max(slices, (tables[t].dim + slice - 1) / slice);
     va.slice_bits = 0;
     while ((1u << va.slice_bits) < slices) ++va.slice_bits;
-    // A hot row takes more than kLongRefs references of its own table, so no
-    // table adds more hot rows than its references allow; a push with no such
-    // table (a few hundred pairs) launches no hot-row kernel and no events.
-    uint64_t hot_rows = 0;
-    for (uint32_t t = 0; t < table_count; ++t)
-      if (DimClass(tables[t].dim) < kClasses - 1) hot_rows += table_refs[t] / (kLongRefs + 1);
     const uint64_t hot_units = hot_rows << va.slice_bits;
     overlap = hot_units != 0 && !(phases & kOneStream) && t_hot_row_overlap;
     if (phases & kPrimary) {
@@ -2218,7 +2227,7 @@ int RunSorted(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, 
           hot_units ? xcd_grid(std::min<uint64_t>(hot_units, long_rows ? kHotGrid : kWideHotGrid)) : 0;
       if (overlap) {
         EPS_HIP_TRY(ThreadOverlap(&ov));
-        EPS_HIP_TRY(Check(hipEventRecord(ov->fork, s), "update fork"));
+        if (!(phases & kForked)) EPS_HIP_TRY(Check(hipEventRecord(ov->fork, s), "update fork"));
         // With the rows beside, the hot rows (the longer part) go out on this
         // stream before the side stream's wait is set up (the wait on a
         // pending event takes ~14 us of host time): they use no class fields
@@ -2345,13 +2354,10 @@ static int PushSetup(const eps_hip_table* tables, const eps_hip_optimizer* optim
   return EPS_HIP_OK;
 }
 
-int eps_hip_push_begin(const eps_hip_table* tables, const eps_hip_optimizer* optimizers,
-                       uint32_t table_count, const eps_hip_push_feature* features,
-                       uint32_t feature_count, void* workspace, uint64_t workspace_bytes,
-                       void* bounds, void* stream) {
-  PushPlan plan;
-  EPS_HIP_TRY(PushSetup(tables, optimizers, table_count, features, feature_count, workspace,
-                        workspace_bytes, bounds, plan));
+// The gradient scan of a push; `done` (if any) is recorded as it completes.
+static int PushScan(const eps_hip_table* tables, uint32_t table_count, const eps_hip_push_feature* features,
+                    uint32_t feature_count, const PushPlan& plan, void* workspace, void* bounds, void* stream,
+                    hipEvent_t done) {
   GuardArgs g{};
   uint64_t blocks = 0;
   auto add = [&](const void* p, uint64_t count, SpanKind kind) {
@@ -2374,7 +2380,17 @@ int eps_hip_push_begin(const eps_hip_table* tables, const eps_hip_optimizer* opt
   add(nullptr, plan.occurrences, kSortedSpan);
   g.ctrl = static_cast<Control*>(workspace);
   g.bounds = static_cast<const Bounds*>(bounds);
-  return LaunchGuard(g, blocks, AsStream(stream));
+  return LaunchGuard(g, blocks, AsStream(stream), done);
+}
+
+int eps_hip_push_begin(const eps_hip_table* tables, const eps_hip_optimizer* optimizers,
+                       uint32_t table_count, const eps_hip_push_feature* features,
+                       uint32_t feature_count, void* workspace, uint64_t workspace_bytes,
+                       void* bounds, void* stream) {
+  PushPlan plan;
+  EPS_HIP_TRY(PushSetup(tables, optimizers, table_count, features, feature_count, workspace,
+                        workspace_bytes, bounds, plan));
+  return PushScan(tables, table_count, features, feature_count, plan, workspace, bounds, stream, nullptr);
 }
 
 static int PushPhase(const eps_hip_table* tables, const eps_hip_optimizer* optimizers,
@@ -2407,18 +2423,41 @@ int eps_hip_push_end(const eps_hip_table* tables, const eps_hip_optimizer* optim
                    workspace_bytes, bounds, stream, kSecond);
 }
 
+// A whole push: scan, update and checked apply from one plan.  Nothing of the
+// caller's can come between the scan and the update, so the side stream is
+// forked from the scan's own completion, without a marker packet behind it
+// (which also holds the row kernels up: 26 tables of ~43,000 references, scan
+// end to row kernel start 11-14 -> 5 us).
+static int PushWhole(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, uint32_t table_count,
+                     const eps_hip_push_feature* features, uint32_t feature_count, void* workspace,
+                     uint64_t workspace_bytes, void* bounds, void* stream, int phases) {
+  PushPlan plan;
+  EPS_HIP_TRY(PushSetup(tables, optimizers, table_count, features, feature_count, workspace,
+                        workspace_bytes, bounds, plan));
+  uint64_t table_refs[EPS_HIP_MAX_TABLES];
+  Overlap* ov = nullptr;
+  if (!(phases & kOneStream) && t_hot_row_overlap &&
+      HotRowBound(tables, table_count, features, feature_count, table_refs)) {
+    EPS_HIP_TRY(ThreadOverlap(&ov));
+    phases |= kForked;
+  }
+  EPS_HIP_TRY(PushScan(tables, table_count, features, feature_count, plan, workspace, bounds, stream,
+                       ov ? ov->fork : nullptr));
+  if (!plan.occurrences) return EPS_HIP_OK;
+  const PushLayout L(plan.occurrences);
+  return RunSorted(tables, optimizers, table_count, features, feature_count, plan, L,
+                   static_cast<uint8_t*>(workspace), false, nullptr, nullptr, 0, static_cast<Bounds*>(bounds),
+                   AsStream(stream), phases);
+}
+
 }  // extern "C"
 
 namespace eps_hip {
 int PushOneStream(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, uint32_t table_count,
                   const eps_hip_push_feature* features, uint32_t feature_count, void* workspace,
                   uint64_t workspace_bytes, void* bounds, void* stream) {
-  EPS_HIP_TRY(eps_hip_push_begin(tables, optimizers, table_count, features, feature_count,
-                                 workspace, workspace_bytes, bounds, stream));
-  EPS_HIP_TRY(PushPhase(tables, optimizers, table_count, features, feature_count, workspace,
-                        workspace_bytes, bounds, stream, kPrimary | kOneStream));
-  return PushPhase(tables, optimizers, table_count, features, feature_count, workspace, workspace_bytes,
-                   bounds, stream, kSecond | kOneStream);
+  return PushWhole(tables, optimizers, table_count, features, feature_count, workspace, workspace_bytes, bounds,
+                   stream, kPrimary | kSecond | kOneStream);
 }
 }  // namespace eps_hip
 
@@ -2428,12 +2467,8 @@ int eps_hip_push(const eps_hip_table* tables, const eps_hip_optimizer* optimizer
                  uint32_t table_count, const eps_hip_push_feature* features,
                  uint32_t feature_count, void* workspace, uint64_t workspace_bytes, void* bounds,
                  void* stream) {
-  EPS_HIP_TRY(eps_hip_push_begin(tables, optimizers, table_count, features, feature_count,
-                                 workspace, workspace_bytes, bounds, stream));
-  EPS_HIP_TRY(eps_hip_push_apply(tables, optimizers, table_count, features, feature_count,
-                                 workspace, workspace_bytes, bounds, stream));
-  return eps_hip_push_end(tables, optimizers, table_count, features, feature_count, workspace,
-                          workspace_bytes, bounds, stream);
+  return PushWhole(tables, optimizers, table_count, features, feature_count, workspace, workspace_bytes, bounds,
+                   stream, kPrimary | kSecond);
 }
 
 int eps_hip_reduce(const eps_hip_table* tables, uint32_t table_count,

@@ -293,8 +293,12 @@ class DeviceShard:
                          1 if s.bounds else 0, lo, hi)
 
     def advance_powers(self, tables):
-        sel = list(set(tables))
-        self.powers[sel] = self.powers[sel] * self._betas[sel]  # fp32 products, as the reference
+        sel = set(tables)
+        if len(sel) == len(self.specs):
+            self.powers *= self._betas  # fp32 products, as the reference
+            return
+        sel = list(sel)
+        self.powers[sel] = self.powers[sel] * self._betas[sel]
 
     # ---- pull ----
     def gather_parts(self, feats, outputs, mean_divide=True):
@@ -317,10 +321,11 @@ class DeviceShard:
             parts = self.gather_parts(feats, outputs, mean_divide)
             return [((GatherPart * len(parts[i:i + MAX_GATHER_PARTS]))(*parts[i:i + MAX_GATHER_PARTS]),
                      len(parts[i:i + MAX_GATHER_PARTS])) for i in range(0, len(parts), MAX_GATHER_PARTS)]
-        chunks = self._cached("gather", list(feats) + list(outputs), build,
-                              (mean_divide, tuple(o.data_ptr() for o in outputs)))
+        chunks = self._cached("gather", [*feats, *outputs], build,
+                              (mean_divide, [o.data_ptr() for o in outputs]))
+        on, gather, flag = _stream(self.torch, stream), lib().eps_hip_gather, _ptr(status)
         for arr, count in chunks:
-            check(lib().eps_hip_gather(arr, count, _ptr(status), _stream(self.torch, stream)))
+            check(gather(arr, count, flag, on))
         return outputs
 
     # ---- push ----
@@ -328,15 +333,20 @@ class DeviceShard:
         """ctypes argument array for these objects, kept for the last few object
         lists seen (an entry holds its objects, so their ids stay unique while it
         lives) and rebuilt when a feature's struct or `extra` has changed."""
-        key = (kind, tuple(map(id, objs)))
+        key = (kind, *map(id, objs))
         hit = self._args_cache.get(key)
-        if hit is not None and hit[1] == extra and all(
-                getattr(a, "_struct", None) is c for a, c in zip(hit[0], hit[2])):
-            return hit[3]
+        if hit is not None and hit[1] == extra:
+            for f, struct in hit[2]:
+                if f._struct is not struct:
+                    break
+            else:
+                return hit[3]
         arr = build()
         if len(self._args_cache) >= 16:
             self._args_cache.pop(next(iter(self._args_cache)))
-        self._args_cache[key] = (list(objs), extra, [getattr(o, "_struct", None) for o in objs], arr)
+        # Only features carry a struct; everything is held, so that ids stay unique.
+        self._args_cache[key] = (list(objs), extra, [(o, o._struct) for o in objs if isinstance(o, DeviceFeature)],
+                                 arr)
         return arr
 
     def _push_args(self, feats):
@@ -366,19 +376,20 @@ class DeviceShard:
         args = (self.tables, self._opts, len(self.specs), arr, len(feats), _ptr(self.wss[slot]), self.ws_bytes,
                 _ptr(self.bounds), _stream(self.torch, stream))
         L = lib()
-        check(L.eps_hip_push_begin(*args))
-        if events:
-            events[0].record(stream)
         if not hot_overlap:
             check(L.eps_hip_set_hot_row_overlap(0))
         try:
-            check(L.eps_hip_push_apply(*args))
+            if events:
+                check(L.eps_hip_push_begin(*args))
+                events[0].record(stream)
+                check(L.eps_hip_push_apply(*args))
+                events[1].record(stream)
+                check(L.eps_hip_push_end(*args))
+            else:
+                check(L.eps_hip_push(*args))
         finally:
             if not hot_overlap:
                 check(L.eps_hip_set_hot_row_overlap(1))
-        if events:
-            events[1].record(stream)
-        check(L.eps_hip_push_end(*args))
         if advance:
             status = self.status(stream, slot=slot)
             if status & STATUS_ERRORS == 0:
