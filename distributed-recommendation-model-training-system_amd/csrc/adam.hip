@@ -2181,7 +2181,8 @@ int RunSorted(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, 
     va.row_bits = plan.row_bits;
     uint64_t table_refs[EPS_HIP_MAX_TABLES];
     const uint64_t hot_rows = HotRowBound(tables, table_count, features, feature_count, table_refs);
-    const bool long_rows = *std::max_element(table_refs, table_refs + table_count) >= kOverlapTableRefs;
+    const uint64_t most_refs = *std::max_element(table_refs, table_refs + table_count);
+    const bool long_rows = most_refs >= kOverlapTableRefs;
     uint64_t vector_occurrences = 0;
     for (uint32_t cls = 0; cls + 1 < kClasses; ++cls) vector_occurrences += plan.class_occurrences[cls];
     // Slice width: pushes with very long hot rows (some table with 65,536 or
@@ -2219,10 +2220,12 @@ int RunSorted(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, 
       // for no event while the longer part runs.  The hot rows are the longer
       // part when some table takes 65,536 or more references (its hottest
       // rows' chains outlast the row runs: 65,536 pairs on one table, hot rows
-      // 80 us against row runs 49 us); otherwise the row runs are.  Both
-      // sides make the guard decision themselves, from the same snapshot, so
-      // they decide the same.
-      const bool rows_beside = overlap && long_rows;
+      // 80 us against row runs 49 us) or a sixteenth of the push's (8 tables
+      // of ~65,000 references, hot rows on the side stream 295 us a step, row
+      // runs there 283; 26 tables of ~43,000 the other way round, 273
+      // against 281); otherwise the row runs are.  Both sides make the guard
+      // decision themselves, from the same snapshot, so they decide the same.
+      const bool rows_beside = overlap && (long_rows || most_refs * 16 >= vector_occurrences);
       const uint64_t hot_blocks =
           hot_units ? xcd_grid(std::min<uint64_t>(hot_units, long_rows ? kHotGrid : kWideHotGrid)) : 0;
       if (overlap) {
