@@ -314,12 +314,22 @@ struct GuardScalars {
   uint64_t refs;       // references summed into one reduced gradient, at most; 0: the prepared count
   uint32_t tables;
 };
-__device__ uint32_t DecideBlock(Control* ctrl, const TableDesc* t, const GuardScalars& gs, uint32_t* s_mode) {
+// What the decision is made from, loaded at once and before the tables are
+// staged, so that a block's start waits for one memory latency and not for one
+// per value.
+struct GuardInputs { uint32_t grad, scale, status, w, m, v, valid; };
+__device__ __forceinline__ GuardInputs LoadGuard(const Control* ctrl) {
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  return GuardInputs{ctrl->src_slots[lane], ctrl->scale_slots[lane], ctrl->prep_status, ctrl->snap[0],
+                     ctrl->snap[1],         ctrl->snap[2],           ctrl->valid_count};
+}
+__device__ uint32_t DecideBlock(Control* ctrl, const GuardInputs& in, const TableDesc* t, const GuardScalars& gs,
+                                uint32_t* s_mode) {
   if (threadIdx.x < kWave) {
     const uint32_t lane = threadIdx.x;
-    const uint32_t gb = WaveMax(ctrl->src_slots[lane]);
-    const uint32_t scale_bits = WaveMax(ctrl->scale_slots[lane]);
-    uint32_t status = ctrl->prep_status;
+    const uint32_t gb = WaveMax(in.grad);
+    const uint32_t scale_bits = WaveMax(in.scale);
+    uint32_t status = in.status;
     uint32_t mode = kFused;
     if (status & (EPS_HIP_STATUS_BAD_INDEX | EPS_HIP_STATUS_BAD_SCALE)) {
       mode = kReject;
@@ -330,9 +340,8 @@ __device__ uint32_t DecideBlock(Control* ctrl, const TableDesc* t, const GuardSc
       status |= EPS_HIP_STATUS_BAD_SCALE;
       mode = kReject;
     } else {
-      const double W = __uint_as_float(ctrl->snap[0]), M = __uint_as_float(ctrl->snap[1]),
-                   V = __uint_as_float(ctrl->snap[2]);
-      const double refs = double(gs.refs ? gs.refs : uint64_t(ctrl->valid_count));
+      const double W = __uint_as_float(in.w), M = __uint_as_float(in.m), V = __uint_as_float(in.v);
+      const double refs = double(gs.refs ? gs.refs : uint64_t(in.valid));
       const double G = GuardGradBound(__uint_as_float(gb), __uint_as_float(scale_bits), refs);
       bool table_safe = true;  // one table per lane
       if (lane < gs.tables) {
@@ -365,11 +374,12 @@ enum Role : uint32_t { kDecide = 0, kFollow = 1, kFallback = 2 };
 
 // Whether this launch has work, and whether it writes (uniform over the
 // block).  s_t must hold the launch's tables; every thread calls it.
-__device__ bool LaunchGate(Control* ctrl, const TableDesc* s_t, const GuardScalars& gs, uint32_t role,
-                           uint32_t* s_mode, bool& write) {
+// `in` (LoadGuard) is used by a deciding launch only.
+__device__ bool LaunchGate(Control* ctrl, const GuardInputs& in, const TableDesc* s_t, const GuardScalars& gs,
+                           uint32_t role, uint32_t* s_mode, bool& write) {
   if (role == kDecide) {
     __syncthreads();  // s_t is staged
-    const uint32_t mode = DecideBlock(ctrl, s_t, gs, s_mode);
+    const uint32_t mode = DecideBlock(ctrl, in, s_t, gs, s_mode);
     write = mode == kFused;
     return mode != kReject;
   }
@@ -732,10 +742,11 @@ __global__ void __launch_bounds__(kBlock) SortedUpdateKernel(FusedArgs a) {
   // The checked apply nearly always has nothing to do.
   if (a.role == kFallback && a.ctrl->mode != kChecked) return;
   __shared__ SortedShared sh;
-  StageSorted(a, sh);
   Control* ctrl = a.ctrl;
+  const GuardInputs in = LoadGuard(ctrl);
+  StageSorted(a, sh);
   bool write = true;
-  if (!LaunchGate(ctrl, sh.t, a.gs, a.role, &sh.mode, write)) return;
+  if (!LaunchGate(ctrl, in, sh.t, a.gs, a.role, &sh.mode, write)) return;
   // The classes' sorted positions, from the workspace, kept inside the push's.
   const uint32_t first = ctrl->class_start[a.cls], last = ctrl->class_start[a.cls_end];
   const uint32_t end = min(last, a.n), start = min(first, end);
@@ -875,10 +886,11 @@ __device__ __forceinline__ const float* RefSource(const float* const* grad, uint
 template <uint32_t kThreads = kBlock>
 __device__ __forceinline__ bool VecPrologue(const VecArgs& a, TableDesc* s_t, const float** s_grad,
                                             uint32_t* s_mode, bool& write, uint64_t* s_rows) {
-  CopyWords<kThreads>(s_t, a.t, sizeof(a.t));
-  CopyWords<kThreads>(s_grad, a.grad, sizeof(a.grad));
-  CopyWords<kThreads>(s_rows, a.grad_rows, sizeof(a.grad_rows));
-  return LaunchGate(a.ctrl, s_t, a.gs, a.role, s_mode, write);
+  const GuardInputs in = LoadGuard(a.ctrl);
+  CopyWords<kThreads>(s_t, a.t, a.tables * uint32_t(sizeof(TableDesc)));
+  CopyWords<kThreads>(s_grad, a.grad, a.features * uint32_t(sizeof(a.grad[0])));
+  CopyWords<kThreads>(s_rows, a.grad_rows, a.features * uint32_t(sizeof(a.grad_rows[0])));
+  return LaunchGate(a.ctrl, in, s_t, a.gs, a.role, s_mode, write);
 }
 
 // One chunk of a hot work unit: positions [cbase, cbase + chunk) of the
@@ -1616,25 +1628,23 @@ struct RunShared {
   uint32_t bad;
 };
 
-// The rows of dimension class `cls` (groups of 2^kLog2G lanes), for block
-// `block` of the `grid` blocks the class has.
+// The rows of a dimension class (groups of 2^kLog2G lanes) at the sorted
+// positions `range`, for block `block` of the `grid` blocks the class has.
 template <uint32_t kLog2G>
 __device__ __forceinline__ void RowRuns(const VecArgs& a, RunShared& sh, const TableDesc* s_t,
-                                        const float* const* s_grad, const uint64_t* s_rows, uint32_t cls,
+                                        const float* const* s_grad, const uint64_t* s_rows, uint2 range,
                                         uint32_t block, uint32_t grid, bool write, RowStats& st) {
   constexpr uint32_t G = 1u << kLog2G;
   constexpr uint32_t ngroups = kBlock / G;
   constexpr uint32_t kWindow = RunPositions(kLog2G);
   constexpr uint32_t kStaged = kWindow + kLongRefs;
   static_assert(kStaged <= kRunPositions + kLongRefs, "row-run window fits its LDS");
-  Control* ctrl = a.ctrl;
   // Safe address for reads a damaged workspace would point elsewhere: the
   // control block and what follows it (far more than a row of 3 x 256 floats).
   const float* safe = reinterpret_cast<const float*>(a.ctrl);
   // The class's sorted positions, from the workspace: kept inside the push's
   // positions, so a damaged workspace cannot send the staging reads past them.
-  const uint32_t first = ctrl->class_start[cls], last = ctrl->class_start[cls + 1];
-  const uint32_t end = min(last, a.n), begin = min(first, end);
+  const uint32_t end = min(range.y, a.n), begin = min(range.x, end);
   const uint32_t row_mask = (1u << a.row_bits) - 1;
   const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const uint32_t lig = threadIdx.x & (G - 1), gid = threadIdx.x >> kLog2G;
@@ -1770,11 +1780,12 @@ RowRunKernel(VecArgs a) {
   __shared__ uint32_t s_mode;
   __shared__ uint64_t s_rows[EPS_HIP_MAX_FEATURES];  // gradient rows per feature
   bool write = false;
+  const uint2 range = make_uint2(a.ctrl->class_start[a.cls], a.ctrl->class_start[a.cls + 1]);
   if (!VecPrologue(a, s_t, s_grad, &s_mode, write, s_rows)) return;
   RowStats st;
   if (threadIdx.x == 0) sh.bad = 0;
   __syncthreads();
-  RowRuns<kLog2G>(a, sh, s_t, s_grad, s_rows, a.cls, blockIdx.x, gridDim.x, write, st);
+  RowRuns<kLog2G>(a, sh, s_t, s_grad, s_rows, range, blockIdx.x, gridDim.x, write, st);
   if (sh.bad) st.err |= EPS_HIP_STATUS_BAD_INDEX;
   FinishBlock(st, a.ctrl, a.bounds, write);
 }
@@ -1791,21 +1802,22 @@ RowRunClassesKernel(VecArgs a) {
   __shared__ uint32_t s_mode;
   __shared__ uint64_t s_rows[EPS_HIP_MAX_FEATURES];
   bool write = false;
-  if (!VecPrologue(a, s_t, s_grad, &s_mode, write, s_rows)) return;
-  RowStats st;
-  if (threadIdx.x == 0) sh.bad = 0;
-  __syncthreads();
   uint32_t cls = 0;
 #pragma unroll
   for (uint32_t c = 1; c + 1 < kClasses; ++c)
     if (a.class_grid[c] && blockIdx.x >= a.class_block[c]) cls = c;
+  const uint2 range = make_uint2(a.ctrl->class_start[cls], a.ctrl->class_start[cls + 1]);
+  if (!VecPrologue(a, s_t, s_grad, &s_mode, write, s_rows)) return;
+  RowStats st;
+  if (threadIdx.x == 0) sh.bad = 0;
+  __syncthreads();
   const uint32_t block = blockIdx.x - a.class_block[cls], grid = a.class_grid[cls];
   switch (cls) {
-    case 0: RowRuns<2>(a, sh, s_t, s_grad, s_rows, 0, block, grid, write, st); break;
-    case 1: RowRuns<3>(a, sh, s_t, s_grad, s_rows, 1, block, grid, write, st); break;
-    case 2: RowRuns<4>(a, sh, s_t, s_grad, s_rows, 2, block, grid, write, st); break;
-    case 3: RowRuns<5>(a, sh, s_t, s_grad, s_rows, 3, block, grid, write, st); break;
-    default: RowRuns<6>(a, sh, s_t, s_grad, s_rows, 4, block, grid, write, st); break;
+    case 0: RowRuns<2>(a, sh, s_t, s_grad, s_rows, range, block, grid, write, st); break;
+    case 1: RowRuns<3>(a, sh, s_t, s_grad, s_rows, range, block, grid, write, st); break;
+    case 2: RowRuns<4>(a, sh, s_t, s_grad, s_rows, range, block, grid, write, st); break;
+    case 3: RowRuns<5>(a, sh, s_t, s_grad, s_rows, range, block, grid, write, st); break;
+    default: RowRuns<6>(a, sh, s_t, s_grad, s_rows, range, block, grid, write, st); break;
   }
   if (sh.bad) st.err |= EPS_HIP_STATUS_BAD_INDEX;
   FinishBlock(st, a.ctrl, a.bounds, write);
@@ -1832,9 +1844,10 @@ __global__ void __launch_bounds__(kBlock) RowUpdateKernel(RowArgs a) {
   __shared__ TableDesc s_t[1];
   __shared__ uint32_t s_mode;
   Control* ctrl = a.ctrl;
+  const GuardInputs in = LoadGuard(ctrl);
   if (threadIdx.x == 0) s_t[0] = a.t;
   bool write = false;
-  if (!LaunchGate(ctrl, s_t, a.gs, a.role, &s_mode, write)) return;
+  if (!LaunchGate(ctrl, in, s_t, a.gs, a.role, &s_mode, write)) return;
   const TableDesc T = a.t;
   const uint32_t dim = T.dim;
   const uint32_t G = kGeneric ? kWave : (1u << a.log2g);
@@ -1871,9 +1884,10 @@ __global__ void __launch_bounds__(kBlock) CsrUpdateKernel(RowArgs a) {
   __shared__ uint32_t s_mode;
   __shared__ __align__(16) float s_tile[kLongTile];
   Control* ctrl = a.ctrl;
+  const GuardInputs in = LoadGuard(ctrl);
   if (threadIdx.x == 0) s_t[0] = a.t;
   bool write = false;
-  if (!LaunchGate(ctrl, s_t, a.gs, a.role, &s_mode, write)) return;
+  if (!LaunchGate(ctrl, in, s_t, a.gs, a.role, &s_mode, write)) return;
   const TableDesc T = a.t;
   const uint32_t dim = T.dim;
   const uint32_t G = kGeneric ? kWave : (1u << a.log2g);

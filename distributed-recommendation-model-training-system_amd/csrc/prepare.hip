@@ -355,8 +355,10 @@ __device__ __forceinline__ void SortScan2(uint32_t& x, uint32_t& y, uint32_t (*s
 // items of the same digit; s_count[digit] (this wavefront's row, zeroed) ends
 // with the wavefront's digit counts.  Items are ranked i = 0, 1, ..., lanes in
 // order within each.
+// (`items`, uniform: later items are not ranked.)
 __device__ __forceinline__ void RankDigits(const uint32_t (&digit)[kSortItems], const bool (&valid)[kSortItems],
-                                           uint32_t bits, uint16_t* s_count, uint32_t (&rank)[kSortItems]) {
+                                           uint32_t bits, uint16_t* s_count, uint32_t (&rank)[kSortItems],
+                                           uint32_t items = kSortItems) {
   const uint32_t lane = threadIdx.x & (kWave - 1);
   const uint64_t lt_mask = (1ull << lane) - 1;
   // Lanes of the item's digit: per bit, the lanes whose bit is this lane's
@@ -371,6 +373,7 @@ __device__ __forceinline__ void RankDigits(const uint32_t (&digit)[kSortItems], 
   for (uint32_t b = 0; b < bits; ++b) {
 #pragma unroll
     for (uint32_t i = 0; i < kSortItems; ++i) {
+      if (i >= items) break;
       const uint32_t mine = uint32_t(__builtin_amdgcn_sbfe(digit[i], b, 1u));  // 0 or ~0
       const uint64_t ones = __ballot(mine != 0);
       lo[i] = __builtin_amdgcn_bitop3_b32(lo[i], uint32_t(ones), mine, 0x90);
@@ -380,6 +383,7 @@ __device__ __forceinline__ void RankDigits(const uint32_t (&digit)[kSortItems], 
 #pragma unroll
   for (uint32_t i = 0; i < kSortItems; ++i) {
     rank[i] = 0;
+    if (i >= items) break;
     if (valid[i]) {
       const uint64_t match = lo[i] | (uint64_t(hi[i]) << 32);
       const uint32_t before = s_count[digit[i]];
@@ -924,16 +928,19 @@ __global__ void __launch_bounds__(kSortBlock) SmallPrepareKernel(SmallArgs a) {
   if (t < 2) s_found[t] = 0;
   if (t == 0) s_valid = 0;
   __syncthreads();
-  // Item i of thread t is occurrence wave * 256 + 64 * i + lane, so that ranks
-  // in (wavefront, item, lane) order are ranks in occurrence order.
+  // Each wavefront has `items` times 64 occurrences, as few as hold the push;
+  // item i of a thread is number 64 * i + lane of its wavefront's, so that
+  // ranks in (wavefront, item, lane) order are ranks in occurrence order.
+  const uint32_t items = (a.n + kSortBlock - 1) / kSortBlock;
+  auto place = [&](uint32_t i) { return (wave * items + i) * kWave + lane; };
   uint32_t key[kSortItems], occ[kSortItems];
   uint64_t slot[kSortItems];
   uint32_t feat[kSortItems], li[kSortItems];
   bool in[kSortItems];
 #pragma unroll
   for (uint32_t i = 0; i < kSortItems; ++i) {
-    occ[i] = wave * (kSortTile / kSortWaves) + i * kWave + lane;
-    in[i] = occ[i] < a.n;
+    occ[i] = place(i);
+    in[i] = i < items && occ[i] < a.n;
     feat[i] = 0;
     for (uint32_t f = 1; f < a.count; ++f) feat[i] += occ[i] >= s_f[f].occ_begin ? 1u : 0u;
     li[i] = occ[i] - s_f[feat[i]].occ_begin;
@@ -993,7 +1000,7 @@ __global__ void __launch_bounds__(kSortBlock) SmallPrepareKernel(SmallArgs a) {
 #pragma unroll
     for (uint32_t i = 0; i < kSortItems; ++i) digit[i] = (key[i] >> a.shift[p]) & (digits - 1);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-    RankDigits(digit, in, a.bits[p], s_count[wave], rank);
+    RankDigits(digit, in, a.bits[p], s_count[wave], rank, items);
     __syncthreads();
     uint32_t total = 0, none = 0;
     if (t < digits) {
@@ -1017,7 +1024,7 @@ __global__ void __launch_bounds__(kSortBlock) SmallPrepareKernel(SmallArgs a) {
     __syncthreads();
 #pragma unroll
     for (uint32_t i = 0; i < kSortItems; ++i) {
-      const uint32_t q = wave * (kSortTile / kSortWaves) + i * kWave + lane;
+      const uint32_t q = place(i);
       if (!in[i]) continue;  // the elements stay the first n
       key[i] = s_key[q];
       occ[i] = s_occ[q];
@@ -1026,7 +1033,7 @@ __global__ void __launch_bounds__(kSortBlock) SmallPrepareKernel(SmallArgs a) {
   const uint32_t n = s_valid;  // valid occurrences: the first n of the sorted ones
 #pragma unroll
   for (uint32_t i = 0; i < kSortItems; ++i) {
-    const uint32_t q = wave * (kSortTile / kSortWaves) + i * kWave + lane;
+    const uint32_t q = place(i);
     if (!in[i]) continue;
     a.keys[q] = key[i];
     if (a.vals) a.vals[q] = occ[i];
@@ -1036,8 +1043,8 @@ __global__ void __launch_bounds__(kSortBlock) SmallPrepareKernel(SmallArgs a) {
   if (n > kLongRefs) {
 #pragma unroll
     for (uint32_t i = 0; i < kSortItems; ++i) {
-      const uint32_t q = wave * (kSortTile / kSortWaves) + i * kWave + lane;
-      const bool hot = q + kLongRefs < n && key[i] < a.hot.generic_key && s_key[q + kLongRefs] == key[i] &&
+      const uint32_t q = place(i);
+      const bool hot = in[i] && q + kLongRefs < n && key[i] < a.hot.generic_key && s_key[q + kLongRefs] == key[i] &&
                        (q == 0 || s_key[q - 1] != key[i]);
       ListHotRows(a.hot, s_key, n, hot ? q : ~0u, key[i]);
     }
