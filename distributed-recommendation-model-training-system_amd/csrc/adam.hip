@@ -431,20 +431,27 @@ __device__ void FinishBlock(const RowStats& st, Control* ctrl, Bounds* bounds, b
 }
 
 // ---------------------------------------------------------------------------
-// Long rows of the drivers below: one row's references summed by a whole block.
+// Long rows of the sorted driver: one row's references summed by a whole block.
 // A group's own loop keeps four gradient rows in flight, so a row of thousands
 // of references would hold its group (and the launch) for a memory latency per
-// four of them.  Here the block's threads load a tile of references together
-// (kLongLoads elements a thread: 8 KiB of floats for the vector shapes), scale
-// them and stage the products in LDS as [reference][column]; thread c then
-// adds column c of the tile in reference order while the next tile's rows and
-// the reference words of the one after it are already on their way.  The sum
-// is the group loop's, bit for bit: acc = acc + src * scale, in order, from +0.
-// A tile takes about 1.3 us, the latency of its rows.  Six tables of dims 10 to
-// 300, 10,600 references each, their longest rows ~1,000: the reduce kernels
-// 1,807 -> 224 us, with every class in one launch.
+// four of them.  Here the block's threads load the gradient rows of a tile of
+// 4,096 products together (2,048 in scalar columns), two tiles ahead, scale
+// them and stage the products in one of two LDS tiles as [reference][column];
+// thread c adds column c of the other tile in reference order meanwhile, its
+// LDS reads a step ahead of its adds.  The sum is the group loop's, bit for
+// bit: acc = acc + src * scale, in order, from +0 (products past the row's end
+// are staged as -0.0f, the identity).  What bounds it is the adding waves:
+// their adds, their share of the staging and a barrier per tile.  Rows past
+// 256 columns take 16-byte loads too, where their alignment allows them.
+// Reduce of six tables of dims 10 to 300, 10,600 references each, the longest
+// rows ~1,000: 328 -> 202 us a dedup and reduce (4-byte loads, one tile of 16
+// references in flight, 80 ns a reference of dim 300 before); four tables of
+// dim 128, 63,000 references each, the longest ~15 %: 486 -> 416; eight of dim
+// 64 without long rows 320 -> 306.  Tiles of 8,192 products add 13 ns a
+// reference of dim 64 instead of 16, but leave two blocks a CU: 387 us for
+// those eight tables.
 constexpr uint32_t kBlockRowRefs = 32;   // rows with more references are summed by the block
-constexpr uint32_t kLongTile = 8192;     // floats of a staged tile
+constexpr uint32_t kLongTile = 4096;     // floats of a staged tile (of two)
 
 // Waits for this wave's LDS accesses, then for the block's other waves: unlike
 // __syncthreads it leaves global loads in flight.
@@ -490,71 +497,160 @@ struct CsrRefs {
   }
 };
 
+// `acc` plus the first `count` rows of a staged tile's column `col`, kPitch
+// floats a row, in order.  Rows from `count` to the next multiple of kAddRows
+// hold -0.0f.
+template <uint32_t kPitch, uint32_t kAddRows>
+__device__ __forceinline__ float AddTile(const float* col, uint32_t count, float acc) {
+  float x[kAddRows], y[kAddRows];
+  auto read = [&](float (&v)[kAddRows], uint32_t r) {
+#pragma unroll
+    for (uint32_t k = 0; k < kAddRows; ++k) v[k] = col[r * kPitch + k * kPitch];
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto add = [&](const float (&v)[kAddRows]) {
+#pragma unroll
+    for (uint32_t k = 0; k < kAddRows; ++k) acc = acc + v[k];
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  read(x, 0);
+#pragma clang loop unroll(disable)
+  for (uint32_t r = 0; r < count; r += 2 * kAddRows) {
+    if (r + kAddRows < count) read(y, r + kAddRows);
+    add(x);
+    if (r + kAddRows >= count) break;
+    if (r + 2 * kAddRows < count) read(x, r + 2 * kAddRows);
+    add(y);
+  }
+  return acc;
+}
+
+// Scratch of BlockRowSum: two staged tiles, and where the references of two
+// groups lie.
+constexpr uint32_t kRefGroup = 128;
+struct RowSumShared {
+  __align__(16) float tile[2][kLongTile];
+  const float* src[2][kRefGroup];
+  float scale[2][kRefGroup];
+};
+
 // `acc` plus references [0, count) of column c0 + threadIdx.x (`acc` when that
-// lies past the dimension; vector shapes: c0 = 0, dim <= 256).  `ok` turns
-// false in any thread that met a reference of no gradient row.  Called by the whole
-// block; `tile` holds kLongTile floats.
+// lies past the dimension).  kVec: rows are 16-byte aligned and dim % 4 == 0.
+// `ok` turns false in any thread that met a reference of no gradient row.
+// Called by the whole block.  A thread each decodes the references of a group
+// of 128 to LDS, a group ahead of the row loads, so that these wait for no
+// reference word: loads return in issue order, and a wait for a word would
+// wait for the rows in flight before it.
 template <bool kVec, class Refs>
-__device__ __forceinline__ float BlockRowSum(float* tile, const Refs& refs, uint32_t count, uint32_t dim,
+__device__ __forceinline__ float BlockRowSum(RowSumShared& sh, const Refs& refs, uint32_t count, uint32_t dim,
                                              uint32_t c0, float acc, bool& ok) {
-  constexpr uint32_t kLongLoads = kVec ? 8 : 16;
-  const uint32_t width = kVec ? dim / 4 : min(dim - c0, kBlock);  // elements of a reference
-  uint32_t log2g = 2;                                             // lanes of a reference
-  while ((1u << log2g) < width) ++log2g;
-  const uint32_t pitch = kVec ? dim : width, cols = pitch;
-  const uint32_t per_step = kBlock >> log2g, tile_refs = kLongLoads * per_step;
-  const uint32_t sub = threadIdx.x >> log2g, e = threadIdx.x & ((1u << log2g) - 1);
-  const bool active = e < width;
-  const uint32_t at = active ? (kVec ? e * 4 : c0 + e) : (kVec ? 0u : c0);
-  float4 x[kLongLoads];
-  float scale[kLongLoads];
-  typename Refs::Word w[kLongLoads];
-  // References past the row's end repeat its last one and are not added.
-  auto load_words = [&](uint32_t base) {
-#pragma unroll
-    for (uint32_t k = 0; k < kLongLoads; ++k) w[k] = refs.Load(min(base + k * per_step + sub, count - 1));
+  constexpr uint32_t kCols = kVec ? 4 : 1;                       // columns of a load
+  constexpr uint32_t kTile = kVec ? kLongTile : kLongTile / 2;   // floats of a tile
+  constexpr uint32_t kLoads = kTile / (kBlock * kCols);          // loads of a thread per tile
+  constexpr uint32_t kDepth = 2;                                 // tiles of rows in flight
+  constexpr uint32_t kAddRows = kVec ? 16 : 8;
+  static_assert(kTile / 256 % kAddRows == 0 && kTile / (kVec ? 32 : 16) <= kRefGroup, "tiles of whole steps, in a group");
+  static_assert(kDepth % 2 == 0, "a slot's tiles lie in one half of the LDS");
+  const uint32_t cols = min(dim - c0, kBlock);
+  uint32_t log2g = kVec ? 3 : 4;                                 // lanes of a reference
+  while ((kCols << log2g) < cols) ++log2g;
+  const uint32_t pitch = kCols << log2g;                         // 16 to 256
+  const uint32_t per_step = kBlock >> log2g, tile_refs = kTile / pitch;
+  const uint32_t sub = threadIdx.x >> log2g, e = (threadIdx.x & ((1u << log2g) - 1)) * kCols;
+  const uint32_t at = e < cols ? e : 0u;
+  struct Rows {
+    float4 x[kLoads];
+    float scale[kLoads];
+  } rows[kDepth];
+  // References past the row's end repeat its last one.
+  typename Refs::Word word;
+  auto load_word = [&](uint32_t group) { word = refs.Load(min(group * kRefGroup + threadIdx.x % kRefGroup, count - 1)); };
+  auto decode = [&](uint32_t group) {
+    if (threadIdx.x >= kRefGroup) return;
+    float scale;
+    sh.src[group % 2][threadIdx.x] = refs.Source(word, c0, scale, ok);
+    sh.scale[group % 2][threadIdx.x] = scale;
   };
-  auto load_rows = [&]() {
-    const float* src[kLongLoads];
+  // The rows of the tile of references from `base` on.
+  auto load_rows = [&](Rows& r, uint32_t base) {
+    const uint32_t half = base / kRefGroup % 2, first = base % kRefGroup + sub;
+    const float* src[kLoads];
 #pragma unroll
-    for (uint32_t k = 0; k < kLongLoads; ++k) src[k] = refs.Source(w[k], at, scale[k], ok);
+    for (uint32_t k = 0; k < kLoads; ++k) {
+      src[k] = sh.src[half][first + k * per_step] + at;
+      r.scale[k] = sh.scale[half][first + k * per_step];
+    }
 #pragma unroll
-    for (uint32_t k = 0; k < kLongLoads; ++k) {
-      if constexpr (kVec) x[k] = Load4(src[k]);
-      else x[k].x = LoadF(src[k]);
+    for (uint32_t k = 0; k < kLoads; ++k) {
+      if constexpr (kVec) r.x[k] = Load4(src[k]);
+      else r.x[k].x = LoadF(src[k]);
     }
   };
-  load_words(0);
-  load_rows();
-  load_words(tile_refs);
-  for (uint32_t base = 0; base < count; base += tile_refs) {
-    LdsBarrier();  // the tile before has been added
-    if (active) {
+  // Their products, into LDS.
+  auto stage = [&](float* tile, const Rows& r, uint32_t base) {
+    if (e >= cols) return;  // (the padding columns are never added)
+    const bool whole = base + tile_refs <= count;
 #pragma unroll
-      for (uint32_t k = 0; k < kLongLoads; ++k) {
-        float* to = tile + (k * per_step + sub) * pitch + (kVec ? e * 4 : e);
-        if constexpr (kVec)
-          *reinterpret_cast<float4*>(to) =
-              make_float4(x[k].x * scale[k], x[k].y * scale[k], x[k].z * scale[k], x[k].w * scale[k]);
-        else
-          *to = x[k].x * scale[k];
-      }
+    for (uint32_t k = 0; k < kLoads; ++k) {
+      float* to = tile + (k * per_step + sub) * pitch + e;
+      const bool in = whole || base + k * per_step + sub < count;
+      const float4 x = r.x[k];
+      const float s = r.scale[k];
+      if constexpr (kVec)
+        *reinterpret_cast<float4*>(to) =
+            make_float4(in ? x.x * s : -0.f, in ? x.y * s : -0.f, in ? x.z * s : -0.f, in ? x.w * s : -0.f);
+      else
+        *to = in ? x.x * s : -0.f;
     }
-    load_rows();
-    load_words(base + 2 * tile_refs);
-    LdsBarrier();
-    if (threadIdx.x < cols) {
-      const uint32_t n = min(tile_refs, count - base);
-      const float* col = tile + threadIdx.x;
-      uint32_t r = 0;
-      for (; r + 16 <= n; r += 16) {
-        float v[16];
+  };
+  // `ahead`: the first reference whose row is not yet asked for.  Where it
+  // starts a group, that group is decoded already; the next one is now, and
+  // the words of the one after it go out before the rows.
+  uint32_t ahead = 0;
+  auto next_rows = [&](Rows& r) {
+    if (ahead % kRefGroup == 0) {
+      decode(ahead / kRefGroup + 1);
+      load_word(ahead / kRefGroup + 2);
+    }
+    load_rows(r, ahead);
+    ahead += tile_refs;
+  };
+  load_word(0);
+  LdsBarrier();  // what an earlier call left in LDS has been read
+  decode(0);
+  load_word(1);
 #pragma unroll
-        for (uint32_t k = 0; k < 16; ++k) v[k] = col[(r + k) * pitch];
+  for (uint32_t d = 0; d < kDepth; ++d) {
+    if (ahead % kRefGroup == 0) LdsBarrier();
+    next_rows(rows[d]);
+  }
+  stage(sh.tile[0], rows[0], 0);
+  LdsBarrier();  // tile 0 is staged, and a group's references decoded (and read)
+  next_rows(rows[0]);
+  // Tile t (of slot d = t % kDepth) is added, and tile t + 1 staged beside it.
+#pragma clang loop unroll(disable)
+  for (uint32_t base = 0; base < count;) {
 #pragma unroll
-        for (uint32_t k = 0; k < 16; ++k) acc = acc + v[k];
+    for (uint32_t d = 0; d < kDepth; ++d) {
+      if (base >= count) break;  // uniform
+      LdsBarrier();  // tile t is staged, tile t - 1 added
+      if (threadIdx.x < cols) {
+        const float* col = sh.tile[d % 2] + threadIdx.x;
+        const uint32_t n = min(tile_refs, count - base);
+        switch (pitch) {
+          case 16: acc = AddTile<16, kAddRows>(col, n, acc); break;
+          case 32: acc = AddTile<32, kAddRows>(col, n, acc); break;
+          case 64: acc = AddTile<64, kAddRows>(col, n, acc); break;
+          case 128: acc = AddTile<128, kAddRows>(col, n, acc); break;
+          default: acc = AddTile<256, kAddRows>(col, n, acc); break;
+        }
       }
-      for (; r < n; ++r) acc = acc + col[r * pitch];
+      base += tile_refs;
+      if (base < count) {
+        Rows& r = rows[(d + 1) % kDepth];
+        stage(sh.tile[(d + 1) % 2], r, base);
+        next_rows(r);
+      }
     }
   }
   return acc;
@@ -577,6 +673,7 @@ struct FusedArgs {
   GuardScalars gs;
   uint32_t row_bits, cls, cls_end, vblocks, role, tables, features;  // classes [cls, cls_end)
   uint32_t n;  // occurrences of the push (sorted positions, occurrence indices)
+  uint32_t wide;  // every gradient array is 16-byte aligned: rows of dim % 4 == 0 too
   uint32_t class_block[kClasses + 1];  // SortedReduceKernel: first block of each class (and the total)
 };
 static_assert(sizeof(FusedArgs) <= 4096, "update arguments fit the kernel-argument segment");
@@ -588,7 +685,7 @@ struct SortedShared {
   uint32_t heads[kBlock];
   uint32_t wave_heads[kBlock / kWave];
   uint32_t mode, bad;
-  __align__(16) float tile[kLongTile];
+  RowSumShared sum;
 };
 
 // The rows whose first position lies in the windows of `ppb` positions that
@@ -709,7 +806,9 @@ __device__ __forceinline__ void SortedRows(const FusedArgs& a, SortedShared& sh,
       const SortedRefs refs{a.rs + row.sb, sh.grad, sh.rows, safe, a.features, T.dim};
       for (uint32_t c0 = 0; c0 < T.dim; c0 += kBlock) {
         bool ok = row.ok;
-        const float acc = BlockRowSum<!kGeneric>(sh.tile, refs, row.se - row.sb, T.dim, c0, 0.f, ok);
+        const bool wide = !kGeneric || (a.wide && T.dim % 4 == 0);  // uniform
+        const float acc = wide ? BlockRowSum<true>(sh.sum, refs, row.se - row.sb, T.dim, c0, 0.f, ok)
+                               : BlockRowSum<false>(sh.sum, refs, row.se - row.sb, T.dim, c0, 0.f, ok);
         if (!ok) sh.bad = 1;
         __syncthreads();
         ok = sh.bad == 0;
@@ -738,7 +837,7 @@ __device__ __forceinline__ void StageSorted(const FusedArgs& a, SortedShared& sh
 
 // Adam of the generic class (one wavefront per row, scalar columns), and the
 // checked apply of every class.
-__global__ void __launch_bounds__(kBlock) SortedUpdateKernel(FusedArgs a) {
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) SortedUpdateKernel(FusedArgs a) {
   // The checked apply nearly always has nothing to do.
   if (a.role == kFallback && a.ctrl->mode != kChecked) return;
   __shared__ SortedShared sh;
@@ -759,7 +858,7 @@ __global__ void __launch_bounds__(kBlock) SortedUpdateKernel(FusedArgs a) {
 
 // Reduced gradients of every class in one launch (class c has the blocks
 // [class_block[c], class_block[c + 1])): the classes' long rows then overlap.
-__global__ void __launch_bounds__(kBlock) SortedReduceKernel(FusedArgs a) {
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) SortedReduceKernel(FusedArgs a) {
   __shared__ SortedShared sh;
   StageSorted(a, sh);
   Control* ctrl = a.ctrl;
@@ -1870,6 +1969,82 @@ __global__ void __launch_bounds__(kBlock) RowUpdateKernel(RowArgs a) {
   FinishBlock(st, ctrl, a.bounds, write);
 }
 
+// CSR packets keep one tile of 8,192 products between two barriers, four
+// blocks a CU: with BlockRowSum's two tiles 43,000 references of dim 64 took 107
+// us a call instead of 122, but 120,000 references of dim 256 310 instead of
+// 263, and without long rows 63,000 of dim 64 88 instead of 83.
+constexpr uint32_t kCsrTile = 8192;  // floats of a staged tile
+
+// `acc` plus references [0, count) of column c0 + threadIdx.x (`acc` when that
+// lies past the dimension; vector shapes: c0 = 0, dim <= 256).  `ok` turns
+// false in any thread that met a reference of no gradient row.  Called by the whole
+// block; `tile` holds kCsrTile floats.
+template <bool kVec>
+__device__ __forceinline__ float CsrRowSum(float* tile, const CsrRefs& refs, uint32_t count, uint32_t dim,
+                                             uint32_t c0, float acc, bool& ok) {
+  constexpr uint32_t kLongLoads = kVec ? 8 : 16;
+  const uint32_t width = kVec ? dim / 4 : min(dim - c0, kBlock);  // elements of a reference
+  uint32_t log2g = 2;                                             // lanes of a reference
+  while ((1u << log2g) < width) ++log2g;
+  const uint32_t pitch = kVec ? dim : width, cols = pitch;
+  const uint32_t per_step = kBlock >> log2g, tile_refs = kLongLoads * per_step;
+  const uint32_t sub = threadIdx.x >> log2g, e = threadIdx.x & ((1u << log2g) - 1);
+  const bool active = e < width;
+  const uint32_t at = active ? (kVec ? e * 4 : c0 + e) : (kVec ? 0u : c0);
+  float4 x[kLongLoads];
+  float scale[kLongLoads];
+  CsrRefs::Word w[kLongLoads];
+  // References past the row's end repeat its last one and are not added.
+  auto load_words = [&](uint32_t base) {
+#pragma unroll
+    for (uint32_t k = 0; k < kLongLoads; ++k) w[k] = refs.Load(min(base + k * per_step + sub, count - 1));
+  };
+  auto load_rows = [&]() {
+    const float* src[kLongLoads];
+#pragma unroll
+    for (uint32_t k = 0; k < kLongLoads; ++k) src[k] = refs.Source(w[k], at, scale[k], ok);
+#pragma unroll
+    for (uint32_t k = 0; k < kLongLoads; ++k) {
+      if constexpr (kVec) x[k] = Load4(src[k]);
+      else x[k].x = LoadF(src[k]);
+    }
+  };
+  load_words(0);
+  load_rows();
+  load_words(tile_refs);
+  for (uint32_t base = 0; base < count; base += tile_refs) {
+    LdsBarrier();  // the tile before has been added
+    if (active) {
+#pragma unroll
+      for (uint32_t k = 0; k < kLongLoads; ++k) {
+        float* to = tile + (k * per_step + sub) * pitch + (kVec ? e * 4 : e);
+        if constexpr (kVec)
+          *reinterpret_cast<float4*>(to) =
+              make_float4(x[k].x * scale[k], x[k].y * scale[k], x[k].z * scale[k], x[k].w * scale[k]);
+        else
+          *to = x[k].x * scale[k];
+      }
+    }
+    load_rows();
+    load_words(base + 2 * tile_refs);
+    LdsBarrier();
+    if (threadIdx.x < cols) {
+      const uint32_t n = min(tile_refs, count - base);
+      const float* col = tile + threadIdx.x;
+      uint32_t r = 0;
+      for (; r + 16 <= n; r += 16) {
+        float v[16];
+#pragma unroll
+        for (uint32_t k = 0; k < 16; ++k) v[k] = col[(r + k) * pitch];
+#pragma unroll
+        for (uint32_t k = 0; k < 16; ++k) acc = acc + v[k];
+      }
+      for (; r < n; ++r) acc = acc + col[r * pitch];
+    }
+  }
+  return acc;
+}
+
 constexpr uint64_t kCsrPiece = 1ull << 30;  // references of one BlockRowSum (it counts in 32 bits)
 
 // CSR rows.  Row r belongs to virtual block r % vblocks: a packet lists its
@@ -1882,7 +2057,7 @@ template <bool kGeneric>
 __global__ void __launch_bounds__(kBlock) CsrUpdateKernel(RowArgs a) {
   __shared__ TableDesc s_t[1];
   __shared__ uint32_t s_mode;
-  __shared__ __align__(16) float s_tile[kLongTile];
+  __shared__ __align__(16) float s_tile[kCsrTile];
   Control* ctrl = a.ctrl;
   const GuardInputs in = LoadGuard(ctrl);
   if (threadIdx.x == 0) s_t[0] = a.t;
@@ -1949,7 +2124,7 @@ __global__ void __launch_bounds__(kBlock) CsrUpdateKernel(RowArgs a) {
       for (uint32_t c0 = 0; c0 < dim; c0 += kBlock) {
         float g = 0.f;
         for (uint64_t at = b; at < e; at += kCsrPiece)
-          g = BlockRowSum<!kGeneric>(s_tile, CsrRefs{a.sources + at, a.scales + at, a.src, dim},
+          g = CsrRowSum<!kGeneric>(s_tile, CsrRefs{a.sources + at, a.scales + at, a.src, dim},
                                      uint32_t(min(e - at, kCsrPiece)), dim, c0, g, ok);
         const uint32_t c = c0 + threadIdx.x;
         if (c < dim) AdamRow1(T, slot, c, g, write, st);
@@ -2169,8 +2344,10 @@ int RunSorted(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, 
     else { o.learning_rate = 1; o.beta1 = 0; o.beta2 = 0; o.epsilon = 1; }
     a.t[k] = MakeTable(tables[t], o);
   }
+  a.wide = 1;
   for (uint32_t f = 0; f < feature_count; ++f) {
     a.grad[f] = features[f].gradients;
+    if (reinterpret_cast<uintptr_t>(features[f].gradients) % 16) a.wide = 0;
     a.grad_rows[f] = features[f].pooling == EPS_HIP_POOL_SEQUENCE ? features[f].occurrences : features[f].bags;
   }
   if (!reduce) {

@@ -99,3 +99,36 @@ def test_compact_long_rows(torch_gpu, pkg, dim):
     assert rc == 0
     got = shard.read_rows(0, at).cpu().numpy().reshape(rows, 3, dim)
     assert_close(got, np.stack([w, m, v], 1), f"compact dim={dim}", strict_ulp=0)
+
+
+@pytest.mark.parametrize("dim", [4, 16, 64, 256, 6, 33, 260, 301])
+def test_reduce_rows_of_several_tiles(torch_gpu, pkg, dim):
+    """Rows of several tiles and groups of 256 references: the last one full, one short and one over."""
+    torch, W, H = torch_gpu, pkg.workloads, pkg.eps_hip
+    rng = np.random.default_rng(3000 + dim)
+    lengths = [33, 63, 64, 65, 127, 129, 255, 256, 257, 511, 513, 768, 769, 1025, 1281]
+    specs = [W.TableSpec(0, dim, 400, seed=3)]
+    feats = [feature_of(W, rng, dim, lengths, specs[0].rows)]
+    print(f"case: dim={dim} row lengths {lengths}", flush=True)
+    check_unique_reduce(torch, W, H, specs, feats)
+
+
+@pytest.mark.parametrize("dim", [260, 300])
+def test_gradients_off_the_vector_grid(torch_gpu, pkg, dim):
+    """Gradient rows four bytes past a 16-byte boundary take the scalar loads: the same bits as aligned ones."""
+    torch, W, H = torch_gpu, pkg.workloads, pkg.eps_hip
+    rng = np.random.default_rng(4000 + dim)
+    f = feature_of(W, rng, dim, [1, 33, 300, 700, 5], 500)
+    states = []
+    for shift in (0, 1):
+        dev = H.DeviceFeature(torch, f)
+        rows = torch.zeros(f.gradient.size + 1, device="cuda")[shift:][: f.gradient.size].view(f.gradient.shape)
+        rows.copy_(dev.gradient)
+        dev.gradient = rows
+        print(f"case: dim={dim} gradients {rows.data_ptr() % 16} bytes past a 16-byte boundary", flush=True)
+        shard = H.DeviceShard(torch, [W.TableSpec(0, dim, 500, seed=6)])
+        shard.init_rows()
+        shard.prepare([dev])
+        assert shard.push([dev]) & H.STATUS_ERRORS == 0
+        states.append(shard.state[0].cpu().numpy())
+    assert np.array_equal(states[0], states[1])
