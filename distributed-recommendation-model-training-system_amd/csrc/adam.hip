@@ -941,6 +941,7 @@ constexpr uint32_t kProducers = kHotBlock / kWave - 1;
 // Sorted positions per row-run window for groups of 2^log2g lanes: about 5
 // rows per group at the usual ~3 references per row.  Wider groups take
 // narrower windows, so a class of wide rows still spreads over many blocks.
+// (RunWindowBits, below: the windows of a push too small to fill the chip.)
 constexpr uint32_t RunPositions(uint32_t log2g) { return log2g <= 4 ? 256u : (log2g == 5 ? 128u : 64u); }
 constexpr uint32_t kRunPositions = RunPositions(2);  // the widest window
 static_assert(kRunPositions <= kBlock, "one thread per staged position finds the row heads");
@@ -960,6 +961,7 @@ struct VecArgs {
   uint32_t n;           // sorted positions of the push (hot-row entries are clamped to them)
   uint32_t spin_limit;  // polls of a hot-row hand-over wait (0: give up at once)
   uint32_t class_block[kClasses], class_grid[kClasses];  // RowRunClassesKernel's blocks per class
+  uint32_t window_bits[kClasses];                        // log2 of each class's row-run window
 };
 static_assert(sizeof(VecArgs) <= 4096, "update arguments fit the kernel-argument segment");
 
@@ -1728,16 +1730,17 @@ struct RunShared {
 };
 
 // The rows of a dimension class (groups of 2^kLog2G lanes) at the sorted
-// positions `range`, for block `block` of the `grid` blocks the class has.
+// positions `range`, for block `block` of the `grid` blocks the class has, in
+// windows of 2^window_bits positions (at most RunPositions(kLog2G)).
 template <uint32_t kLog2G>
 __device__ __forceinline__ void RowRuns(const VecArgs& a, RunShared& sh, const TableDesc* s_t,
                                         const float* const* s_grad, const uint64_t* s_rows, uint2 range,
-                                        uint32_t block, uint32_t grid, bool write, RowStats& st) {
+                                        uint32_t block, uint32_t grid, uint32_t window_bits, bool write,
+                                        RowStats& st) {
   constexpr uint32_t G = 1u << kLog2G;
   constexpr uint32_t ngroups = kBlock / G;
-  constexpr uint32_t kWindow = RunPositions(kLog2G);
-  constexpr uint32_t kStaged = kWindow + kLongRefs;
-  static_assert(kStaged <= kRunPositions + kLongRefs, "row-run window fits its LDS");
+  static_assert(RunPositions(kLog2G) <= kRunPositions, "row-run window fits its LDS");
+  const uint32_t window = 1u << window_bits;
   // Safe address for reads a damaged workspace would point elsewhere: the
   // control block and what follows it (far more than a row of 3 x 256 floats).
   const float* safe = reinterpret_cast<const float*>(a.ctrl);
@@ -1755,10 +1758,10 @@ __device__ __forceinline__ void RowRuns(const VecArgs& a, RunShared& sh, const T
   // all their references.  Rows that straddle a cut belong to the range
   // holding their first position.
   const uint32_t xcd = block % kXcds, per_xcd = grid / kXcds;
-  const uint32_t span = ((end - begin + kXcds - 1) / kXcds + kWindow - 1) / kWindow * kWindow;
+  const uint32_t span = ((end - begin + kXcds - 1) / kXcds + window - 1) >> window_bits << window_bits;
   const uint32_t xbegin = min(begin + xcd * span, end), xend = min(xbegin + span, end);
-  for (uint32_t p0 = xbegin + (block / kXcds) * kWindow; p0 < xend; p0 += per_xcd * kWindow) {
-    const uint32_t p1 = min(p0 + kWindow, xend);
+  for (uint32_t p0 = xbegin + (block / kXcds) * window; p0 < xend; p0 += per_xcd * window) {
+    const uint32_t p1 = min(p0 + window, xend);
     const uint32_t lim = min(p1 + kLongRefs, end);
     const uint32_t staged = lim - p0;
     __syncthreads();  // previous iteration's readers are done
@@ -1884,7 +1887,8 @@ RowRunKernel(VecArgs a) {
   RowStats st;
   if (threadIdx.x == 0) sh.bad = 0;
   __syncthreads();
-  RowRuns<kLog2G>(a, sh, s_t, s_grad, s_rows, range, blockIdx.x, gridDim.x, write, st);
+  RowRuns<kLog2G>(a, sh, s_t, s_grad, s_rows, range, blockIdx.x, gridDim.x, a.window_bits[kLog2G - 2], write,
+                  st);
   if (sh.bad) st.err |= EPS_HIP_STATUS_BAD_INDEX;
   FinishBlock(st, a.ctrl, a.bounds, write);
 }
@@ -1911,12 +1915,13 @@ RowRunClassesKernel(VecArgs a) {
   if (threadIdx.x == 0) sh.bad = 0;
   __syncthreads();
   const uint32_t block = blockIdx.x - a.class_block[cls], grid = a.class_grid[cls];
+  const uint32_t bits = a.window_bits[cls];
   switch (cls) {
-    case 0: RowRuns<2>(a, sh, s_t, s_grad, s_rows, range, block, grid, write, st); break;
-    case 1: RowRuns<3>(a, sh, s_t, s_grad, s_rows, range, block, grid, write, st); break;
-    case 2: RowRuns<4>(a, sh, s_t, s_grad, s_rows, range, block, grid, write, st); break;
-    case 3: RowRuns<5>(a, sh, s_t, s_grad, s_rows, range, block, grid, write, st); break;
-    default: RowRuns<6>(a, sh, s_t, s_grad, s_rows, range, block, grid, write, st); break;
+    case 0: RowRuns<2>(a, sh, s_t, s_grad, s_rows, range, block, grid, bits, write, st); break;
+    case 1: RowRuns<3>(a, sh, s_t, s_grad, s_rows, range, block, grid, bits, write, st); break;
+    case 2: RowRuns<4>(a, sh, s_t, s_grad, s_rows, range, block, grid, bits, write, st); break;
+    case 3: RowRuns<5>(a, sh, s_t, s_grad, s_rows, range, block, grid, bits, write, st); break;
+    default: RowRuns<6>(a, sh, s_t, s_grad, s_rows, range, block, grid, bits, write, st); break;
   }
   if (sh.bad) st.err |= EPS_HIP_STATUS_BAD_INDEX;
   FinishBlock(st, a.ctrl, a.bounds, write);
@@ -2269,6 +2274,27 @@ constexpr uint64_t kHotGrid = 512;      // two blocks per CU (LDS: four 17 KiB t
 // step of pull + push, 256 blocks 236, 512 blocks 240).
 constexpr uint64_t kWideHotGrid = 256;
 
+// log2 of each class's row-run window.  A push of fewer than kRunBlocks windows
+// (two a CU) halves them until it has as many, down to one position a lane
+// group: with whole windows a group works through several rows, one memory
+// latency after another, while CUs stand idle.  256 pairs of dim 32 34.3 ->
+// 31.2 us a step; eight tables of 1,500 references, dims 16 to 256, 107 -> 94; four of
+// 4,400 of dim 128 112 -> 97; 20,000 pairs of dim 256 109 -> 106.  (Up to 1,024
+// windows: four tables of 22,000 references of dim 4 97 -> 101, since every
+// window stages kLongRefs positions of look-ahead.)
+constexpr uint64_t kRunBlocks = 512;
+void RunWindowBits(const std::array<uint64_t, kClasses>& positions, uint32_t* bits) {
+  uint64_t windows = 0;
+  for (uint32_t c = 0; c + 1 < kClasses; ++c) windows += (positions[c] + RunPositions(c + 2) - 1) / RunPositions(c + 2);
+  uint32_t halvings = 0;
+  while (windows << halvings < kRunBlocks && halvings < 6) ++halvings;
+  for (uint32_t c = 0; c + 1 < kClasses; ++c) {
+    const uint32_t window = std::max(RunPositions(c + 2) >> halvings, kBlock >> (c + 2));
+    bits[c] = 0;
+    while ((1u << bits[c]) < window) ++bits[c];
+  }
+}
+
 template <uint32_t kLog2G>
 int LaunchRowRun(unsigned grid, const VecArgs& a, hipStream_t s, hipEvent_t done) {
   LaunchRecording(RowRunKernel<kLog2G>, dim3(grid), dim3(kBlock), s, done, a);
@@ -2446,14 +2472,14 @@ int RunSorted(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, 
       // for all of them when there are several.
       uint32_t present = 0;
       uint64_t total_blocks = 0;
+      RunWindowBits(plan.class_occurrences, va.window_bits);
       for (uint32_t cls = 0; cls + 1 < kClasses; ++cls) {
         va.class_block[cls] = uint32_t(total_blocks);
         va.class_grid[cls] = 0;
         if (!plan.class_occurrences[cls]) continue;
-        const uint64_t blocks = xcd_grid(std::min<uint64_t>(
-            std::max<uint64_t>(1, (plan.class_occurrences[cls] + RunPositions(cls + 2) - 1) /
-                                      RunPositions(cls + 2)),
-            kVectorGrid));
+        const uint64_t window = 1ull << va.window_bits[cls];
+        const uint64_t blocks =
+            xcd_grid(std::min<uint64_t>((plan.class_occurrences[cls] + window - 1) / window, kVectorGrid));
         va.class_grid[cls] = uint32_t(blocks);
         total_blocks += blocks;
         ++present;
