@@ -414,6 +414,12 @@ __global__ void InitRowsKernel(float* state, uint32_t dim, uint64_t first, uint6
 }
 
 // ScatterState (src/cuda/cache_backend.cu:69-74): packed [w|m|v] rows -> slots.
+// From pinned host memory the host link bounds it, and the link is slower with
+// more reads waiting on it than fill it: 4,096 rows of dim 64 (3.1 MB) take 128
+// us with 8 blocks of 16-byte loads, 68 with 16, 60 with 32 or 64, 64 with 256
+// and 79 with 768, a thread a load (a copy of that size 69).  Loads of 4 bytes
+// keep a thread a load.
+constexpr unsigned kHostReadGrid = 64;
 __global__ void ScatterRowsKernel(float* state, uint32_t dim, const uint64_t* slots,
                                   const float* packed, uint64_t count, Bounds* bounds) {
   uint32_t bw = 0, bm = 0, bv = 0;
@@ -641,10 +647,13 @@ int eps_hip_scatter_rows(const eps_hip_table* t, const uint64_t* slots, const fl
   if (!count) return EPS_HIP_OK;
   if (!slots || !packed) return Fail(EPS_HIP_INVALID_ARGUMENT, "null scatter buffers");
   const void* source = nullptr;
-  EPS_HIP_TRY(DeviceAddress(packed, &source));
+  bool host = false;
+  EPS_HIP_TRY(DeviceAddress(packed, &source, &host));
   packed = static_cast<const float*>(source);
-  const uint64_t work = (t->dim % 4 == 0) ? count * t->dim * 3 / 4 : count * t->dim * 3;
-  hipLaunchKernelGGL(ScatterRowsKernel, dim3(GridFor(work)), dim3(kBlock), 0, AsStream(stream),
+  const bool vec = t->dim % 4 == 0;
+  const uint64_t work = vec ? count * t->dim * 3 / 4 : count * t->dim * 3;
+  const unsigned grid = host && vec ? GridFor(work, kHostReadGrid) : GridFor(work);
+  hipLaunchKernelGGL(ScatterRowsKernel, dim3(grid), dim3(kBlock), 0, AsStream(stream),
                      t->state, t->dim, slots, packed, count, static_cast<Bounds*>(bounds));
   EPS_HIP_LAUNCHED("scatter rows");
   return EPS_HIP_OK;
