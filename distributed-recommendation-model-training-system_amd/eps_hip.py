@@ -344,9 +344,11 @@ class DeviceShard:
         arr = build()
         if len(self._args_cache) >= 16:
             self._args_cache.pop(next(iter(self._args_cache)))
-        # Only features carry a struct; everything is held, so that ids stay unique.
-        self._args_cache[key] = (list(objs), extra, [(o, o._struct) for o in objs if isinstance(o, DeviceFeature)],
-                                 arr)
+        # Everything is held, so that ids stay unique.  A feature's struct is its
+        # version: it is made here also for one that is only looked up, since
+        # an assignment drops it (to None) and the next use makes another.
+        self._args_cache[key] = (list(objs), extra,
+                                 [(o, o.push_struct()) for o in objs if isinstance(o, DeviceFeature)], arr)
         return arr
 
     def _push_args(self, feats):
