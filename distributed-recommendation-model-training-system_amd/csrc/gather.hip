@@ -67,9 +67,8 @@ struct GatherArgs {
 };
 static_assert(sizeof(GatherArgs) <= 4096, "gather arguments fit the kernel-argument segment");
 
-// Slot of occurrence `i` (or kHole); range failures are reported and skipped.
-__device__ __forceinline__ uint64_t ResolveSlot(const GatherDesc& d, uint64_t i, bool& bad) {
-  uint64_t idx = d.indices[i];
+// Slot of an occurrence's index (or kHole); range failures are reported and skipped.
+__device__ __forceinline__ uint64_t ResolveSlot(const GatherDesc& d, uint64_t idx, bool& bad) {
   if (idx == kHole) return kHole;
   if (d.remap) {
     if (idx >= d.remap_count) { bad = true; return kHole; }
@@ -143,33 +142,58 @@ __device__ __forceinline__ uint64_t Uniform(uint64_t x) {
   return lo | (uint64_t(hi) << 32);
 }
 
+// Orders a wavefront's LDS accesses before and after it (they are performed in
+// order: the compiler is held).
+__device__ __forceinline__ void WaveLdsFence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
+// Stages the row of one occurrence, of index `idx`, as entry `k`.
+__device__ __forceinline__ void StageRow(const GatherDesc& d, GatherShared& sh, uint32_t k, uint64_t idx, bool& bad) {
+  const uint64_t slot = ResolveSlot(d, idx, bad);
+  if (d.buffer_bytes) sh.at32[k] = slot == kHole ? kBufferOutside : uint32_t(slot * d.stride * 4);
+  else sh.at64[k] = slot == kHole ? kHole : slot * d.stride * 4;
+}
+
 // Stages occurrences [first, first + n) of a part (n <= kIdCap): the remap and
 // the range check are done once per occurrence.
 __device__ __forceinline__ void StageOccurrences(const GatherDesc& d, GatherShared& sh, uint64_t first, uint32_t n,
                                                  bool& bad) {
   for (uint32_t k = threadIdx.x; k < n; k += kBlock) {
-    const uint64_t slot = ResolveSlot(d, first + k, bad);
-    if (d.buffer_bytes) sh.at32[k] = slot == kHole ? kBufferOutside : uint32_t(slot * d.stride * 4);
-    else sh.at64[k] = slot == kHole ? kHole : slot * d.stride * 4;
+    StageRow(d, sh, k, d.indices[first + k], bad);
     if (d.pooling == EPS_HIP_POOL_WEIGHTED_SUM) sh.weight[k] = d.weights[first + k];
   }
 }
 
 // The output rows row0 .. row0 + nrows of a pooled part, a group of 2^log2g
 // lanes per row (at most one row a group) and V columns a lane.  The block's
-// occurrences [occ_begin, occ_end) are staged kIdCap at a time, usually once.
+// occurrences [occ_begin, occ_end) are staged at once when there are up to
+// kIdCap of them.  In a block with more, each group stages its own bag's, its
+// share of the entries (four a lane) at a time; when one bag has them all
+// (kOneBag), the whole block stages them for its group, kIdCap at a time.
 // Each is staged as the offset of its row, so that a load costs a lane one LDS
 // read and an add instead of a 64-bit multiply per row and lane, which bound
 // the launch: 26 x 4,096 bags of 1-20 rows of dim 64, 46 -> 41 us; 4 x 262,144
 // bags of 32 rows of dim 128 (38 GB of state, past a buffer range), 1,775 ->
 // 1,071 us.
-template <uint32_t V, bool kWeighted, bool kBuffered>
+template <uint32_t V, bool kWeighted, bool kBuffered, bool kOneBag>
 __device__ __forceinline__ void PoolRows(const GatherDesc& d, GatherShared& sh, uint64_t row0, uint32_t nrows,
-                                         uint64_t occ_begin, uint64_t occ_end, bool& bad) {
+                                         uint64_t occ_begin, uint64_t occ_end, bool none, bool& bad) {
   const uint32_t G = 1u << d.log2g;
   const uint32_t lig = threadIdx.x & (G - 1);
   const uint32_t r = threadIdx.x >> d.log2g;
-  const bool once = occ_end - occ_begin <= kIdCap;
+  const bool once = !kOneBag && occ_end - occ_begin <= kIdCap;  // (uniform over the block)
+  if (once) {
+    StageOccurrences(d, sh, occ_begin, uint32_t(occ_end - occ_begin), bad);
+    __syncthreads();
+  }
+  // A mean's divisor (0: none), asked for before the rows.
+  float divisor = 0.f;
+  if (d.pooling == EPS_HIP_POOL_MEAN && d.lengths && r < nrows) divisor = (float)d.lengths[row0 + r];
+  constexpr uint32_t kOwn = kIdCap / kBlock;  // entries of a lane
+  const uint32_t room = kOwn << d.log2g;      // entries of a group
   // One step for rows of up to 64 * V columns.
   for (uint32_t c0 = 0; c0 < d.dim; c0 += G * V) {
     const uint32_t c = c0 + lig * V;
@@ -184,18 +208,9 @@ __device__ __forceinline__ void PoolRows(const GatherDesc& d, GatherShared& sh, 
         else acc.c[k] += x.c[k];
       }
     };
-    for (uint64_t chunk = occ_begin; chunk < occ_end; chunk += kIdCap) {
-      const uint32_t n = uint32_t(min<uint64_t>(kIdCap, occ_end - chunk));
-      if (c0 == 0 || !once) {
-        if (c0 != 0 || chunk != occ_begin) __syncthreads();  // the chunk before has been added
-        StageOccurrences(d, sh, chunk, n, bad);
-        __syncthreads();
-      }
-      // The row's staged occurrences [first, e).
-      if (r >= nrows || !active) continue;
-      const uint64_t from = max(sh.off[r], chunk), to = min(sh.off[r + 1], chunk + n);
-      if (from >= to) continue;
-      const uint32_t first = uint32_t(from - chunk), e = uint32_t(to - chunk);
+    // Adds the staged entries [first, e), kBatch rows in flight.
+    auto add_staged = [&](auto batch, uint32_t first, uint32_t e) {
+      constexpr uint32_t kBatch = decltype(batch)::value;
       if constexpr (kBuffered) {
         // Through the buffer range: occurrences past the bag and holes read
         // zeros without a memory request, and adding them (weighted: zero
@@ -204,47 +219,90 @@ __device__ __forceinline__ void PoolRows(const GatherDesc& d, GatherShared& sh, 
         // is added.
         const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<float*>(d.source), (short)0, int(d.buffer_bytes), kBufferWord3);
-        for (uint32_t pos = first; pos < e; pos += kGatherBatch) {
-          Columns<V> v[kGatherBatch];
-          uint32_t at[kGatherBatch];
+        for (uint32_t pos = first; pos < e; pos += kBatch) {
+          Columns<V> v[kBatch];
+          uint32_t at[kBatch];
 #pragma unroll
-          for (uint32_t u = 0; u < kGatherBatch; ++u) at[u] = sh.at32[pos + u];
+          for (uint32_t u = 0; u < kBatch; ++u) at[u] = sh.at32[pos + u];
 #pragma unroll
-          for (uint32_t u = 0; u < kGatherBatch; ++u) {
+          for (uint32_t u = 0; u < kBatch; ++u) {
             at[u] = pos + u < e ? at[u] : kBufferOutside;
             v[u] = LoadColumns<V>(rsrc, at[u] + c * 4);
           }
 #pragma unroll
-          for (uint32_t u = 0; u < kGatherBatch; ++u)
+          for (uint32_t u = 0; u < kBatch; ++u)
             add(v[u], !kWeighted ? 1.f : at[u] != kBufferOutside ? sh.weight[pos + u] : 0.f);
         }
       } else if (d.source_rows) {  // (without rows every occurrence is a hole)
         // No branch around a load: a hole or a position past the bag reads
         // row 0 and is dropped.
         const char* source = reinterpret_cast<const char*>(d.source + c);
-        for (uint32_t pos = first; pos < e; pos += kGatherBatch) {
-          Columns<V> v[kGatherBatch];
-          bool ok[kGatherBatch];
+        for (uint32_t pos = first; pos < e; pos += kBatch) {
+          Columns<V> v[kBatch];
+          bool ok[kBatch];
 #pragma unroll
-          for (uint32_t u = 0; u < kGatherBatch; ++u) {
+          for (uint32_t u = 0; u < kBatch; ++u) {
             const uint64_t at = sh.at64[min(pos + u, e - 1)];
             ok[u] = pos + u < e && at != kHole;
             v[u] = LoadColumns<V>(reinterpret_cast<const float*>(source + (ok[u] ? at : 0)));
           }
 #pragma unroll
-          for (uint32_t u = 0; u < kGatherBatch; ++u)
+          for (uint32_t u = 0; u < kBatch; ++u)
             if (ok[u]) add(v[u], kWeighted ? sh.weight[pos + u] : 1.f);
         }
       }
+    };
+    if constexpr (kOneBag) {
+      for (uint64_t chunk = occ_begin; chunk < occ_end; chunk += kIdCap) {
+        const uint32_t n = uint32_t(min<uint64_t>(kIdCap, occ_end - chunk));
+        __syncthreads();  // the chunk before has been added
+        StageOccurrences(d, sh, chunk, n, bad);
+        __syncthreads();
+        if (active && sh.off[r] < sh.off[r + 1]) add_staged(std::integral_constant<uint32_t, kGatherBatch>{}, 0u, n);
+      }
+    } else if (once) {
+      // (Kept inside the staged entries, whatever the offsets.)
+      const uint64_t from = max(sh.off[r], occ_begin), to = min(sh.off[r + 1], occ_end);
+      if (active && from < to)
+        add_staged(std::integral_constant<uint32_t, kGatherBatch>{}, uint32_t(from - occ_begin),
+                   uint32_t(to - occ_begin));
+    } else if (!none) {
+      // A group lies in one wavefront, whose LDS accesses are performed in
+      // order, so no barrier comes between the groups: with the block staging
+      // kIdCap occurrences between two barriers, one bag of a block was added
+      // at a time (1,000 bags of 1,500 rows of dim 64, 16 bags a block: 1,036
+      // us, 128 so; 64 of 2,000 of dim 4, a block: 3,860, 257 so).  A block's
+      // only bag is better off with that (20,000 rows of dim 3: 0.99 ms, its
+      // group alone 2.65; 500,000 of dim 64: 23, 29).
+      const uint32_t entry = r * room;
+      for (uint64_t from = sh.off[r]; from < sh.off[r + 1]; from += room) {
+        const uint32_t n = uint32_t(min<uint64_t>(room, sh.off[r + 1] - from));
+        uint64_t idx[kOwn];
+#pragma unroll
+        for (uint32_t k = 0; k < kOwn; ++k) idx[k] = d.indices[from + min(k * G + lig, n - 1)];
+#pragma unroll
+        for (uint32_t k = 0; k < kOwn; ++k) {
+          const uint32_t at = k * G + lig;
+          if (at < n) StageRow(d, sh, entry + at, idx[k], bad);
+        }
+        if constexpr (kWeighted) {
+          __builtin_amdgcn_sched_barrier(0);  // (all at once, they cost the launch a wavefront a SIMD)
+          float weight[kOwn];
+#pragma unroll
+          for (uint32_t k = 0; k < kOwn; ++k) weight[k] = d.weights[from + min(k * G + lig, n - 1)];
+#pragma unroll
+          for (uint32_t k = 0; k < kOwn; ++k)
+            if (k * G + lig < n) sh.weight[entry + k * G + lig] = weight[k];
+        }
+        WaveLdsFence();
+        if (active) add_staged(std::integral_constant<uint32_t, V == 4 && kWeighted ? 6 : kGatherBatch>{}, entry, entry + n);
+        WaveLdsFence();  // the entries have been read
+      }
     }
     if (r >= nrows || !active) continue;
-    if (d.pooling == EPS_HIP_POOL_MEAN && d.lengths) {
-      const uint64_t len = d.lengths[row0 + r];
-      if (len) {
-        const float f = (float)len;
+    if (divisor != 0.f) {
 #pragma unroll
-        for (uint32_t k = 0; k < V; ++k) acc.c[k] = acc.c[k] / f;
-      }
+      for (uint32_t k = 0; k < V; ++k) acc.c[k] = acc.c[k] / divisor;
     }
     StoreColumns<V>(d.output + (row0 + r) * d.dim + c, acc);
   }
@@ -313,7 +371,8 @@ __global__ void __launch_bounds__(kBlock) GatherKernel(GatherArgs args) {
     else if (d.width == 2) CopyRows<2>(d, sh, row0, nrows);
     else CopyRows<1>(d, sh, row0, nrows);
   } else {
-    for (uint32_t r = threadIdx.x; r <= nrows; r += kBlock) sh.off[r] = d.offsets[row0 + r];
+    // (Groups past the rows have empty bags.)
+    for (uint32_t r = threadIdx.x; r <= kBlock / 4; r += kBlock) sh.off[r] = d.offsets[row0 + min(r, nrows)];
     __syncthreads();
     const uint64_t occ_begin = Uniform(sh.off[0]);
     // A part without indices has no occurrences (every bag empty): nothing is
@@ -321,9 +380,16 @@ __global__ void __launch_bounds__(kBlock) GatherKernel(GatherArgs args) {
     const bool none = d.indices == nullptr;
     if (none && sh.off[nrows] != occ_begin && threadIdx.x == 0) sh.bad = 1;
     const uint64_t occ_end = none ? occ_begin : Uniform(sh.off[nrows]);
+    const bool one_bag = occ_end - occ_begin > kIdCap && !none &&
+                         __syncthreads_or(sh.off[threadIdx.x & (kBlock / 4 - 1)] == occ_begin &&
+                                          sh.off[(threadIdx.x & (kBlock / 4 - 1)) + 1] == occ_end);
     auto pool = [&](auto v, auto weighted, auto through) {
-      PoolRows<decltype(v)::value, decltype(weighted)::value, decltype(through)::value>(d, sh, row0, nrows, occ_begin,
-                                                                                       occ_end, bad);
+      auto rows = [&](auto one) {
+        PoolRows<decltype(v)::value, decltype(weighted)::value, decltype(through)::value, decltype(one)::value>(
+            d, sh, row0, nrows, occ_begin, occ_end, none, bad);
+      };
+      if (one_bag) rows(std::true_type{});
+      else rows(std::false_type{});
     };
     auto with_width = [&](auto weighted, auto through) {
       if (d.width == 4) pool(std::integral_constant<uint32_t, 4>{}, weighted, through);
