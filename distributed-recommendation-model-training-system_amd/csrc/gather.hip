@@ -194,6 +194,32 @@ __device__ __forceinline__ void PoolRows(const GatherDesc& d, GatherShared& sh, 
   if (d.pooling == EPS_HIP_POOL_MEAN && d.lengths && r < nrows) divisor = (float)d.lengths[row0 + r];
   constexpr uint32_t kOwn = kIdCap / kBlock;  // entries of a lane
   const uint32_t room = kOwn << d.log2g;      // entries of a group
+  // A bag of one row of several steps is a copy of it (through +0.0f): its
+  // steps' loads go out together, without the rest of a batch (10,000 bags of
+  // dim 258, 12.7 us as sums, 7.8 so; of dim 300, 10.4 and 7.8).
+  const uint64_t first = sh.off[r] - occ_begin;
+  if (once && G * V < d.dim && r < nrows && sh.off[r + 1] - sh.off[r] == 1 && first < kIdCap &&
+      (kBuffered || sh.at64[first] != kHole)) {
+    const uint32_t at = kBuffered ? sh.at32[first] : 0u;  // (a hole reads zeros)
+    const float weight = !kWeighted ? 1.f : kBuffered && at == kBufferOutside ? 0.f : sh.weight[first];
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(d.source), (short)0, int(d.buffer_bytes), kBufferWord3);
+    const float* row = d.source + (kBuffered ? 0 : sh.at64[first] / 4);
+    float* out = d.output + (row0 + r) * d.dim;
+#pragma unroll 4
+    for (uint32_t c = lig * V; c < d.dim; c += G * V) {
+      Columns<V> x;
+      if constexpr (kBuffered) x = LoadColumns<V>(rsrc, at + c * 4);
+      else x = LoadColumns<V>(row + c);
+#pragma unroll
+      for (uint32_t q = 0; q < V; ++q) {
+        x.c[q] = 0.f + (kWeighted ? x.c[q] * weight : x.c[q]);
+        if (divisor != 0.f) x.c[q] = x.c[q] / divisor;
+      }
+      StoreColumns<V>(out + c, x);
+    }
+    return;
+  }
   // One step for rows of up to 64 * V columns.
   for (uint32_t c0 = 0; c0 < d.dim; c0 += G * V) {
     const uint32_t c = c0 + lig * V;

@@ -81,6 +81,14 @@ def test_one_bag_of_a_block(torch_gpu, pkg, dim, pooling):
         check(torch_gpu, W, H, dim, pooling, rng, rows=100, lengths=lengths)
 
 
+@pytest.mark.parametrize("dim", [256, 257, 258, 260, 300, 1028, 1030, 16_384, 16_385, 16_386, 16_388])
+@pytest.mark.parametrize("pooling", [0, 1, 3])
+def test_bags_of_one_row(torch_gpu, pkg, dim, pooling):
+    """Bags of at most one occurrence, holes among them: copies where a row is wider than a wavefront's columns."""
+    check(torch_gpu, pkg.workloads, pkg.eps_hip, dim, pooling, np.random.default_rng(dim * 17 + pooling), rows=60,
+          bags=45, max_len=1, holes=0.3)
+
+
 # The last dimension read through a 32-bit buffer range, and the first ones past it: loads of 1, 2 and 4 floats.
 @pytest.mark.parametrize("dim", [16_384, 16_385, 16_386, 16_388])
 @pytest.mark.parametrize("pooling", [0, 1, 2, 3])
