@@ -2437,12 +2437,15 @@ int RunSorted(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, 
       // for no event while the longer part runs.  The hot rows are the longer
       // part when some table takes 65,536 or more references (its hottest
       // rows' chains outlast the row runs: 65,536 pairs on one table, hot rows
-      // 80 us against row runs 49 us) or a sixteenth of the push's (8 tables
-      // of ~65,000 references, hot rows on the side stream 295 us a step, row
-      // runs there 283; 26 tables of ~43,000 the other way round, 273
-      // against 281); otherwise the row runs are.  Both sides make the guard
-      // decision themselves, from the same snapshot, so they decide the same.
-      const bool rows_beside = overlap && (long_rows || most_refs * 16 >= vector_occurrences);
+      // 80 us against row runs 49 us); otherwise the row runs are.  (Below that
+      // it turns on the skew, which the host does not know: with the row runs
+      // on the side stream, eight tables of 64,000 references take 109 us a
+      // push instead of 115 when their ids are Zipf of 1.05 and 115 instead of
+      // 134 at 1.2, but fourteen of 20,000 take 89 instead of 71, eight of
+      // 43,000 94 instead of 86, and two of 64,000 uniform ids 74 instead of
+      // 62.)  Both sides make the guard decision themselves, from the same
+      // snapshot, so they decide the same.
+      const bool rows_beside = overlap && long_rows;
       const uint64_t hot_blocks =
           hot_units ? xcd_grid(std::min<uint64_t>(hot_units, long_rows ? kHotGrid : kWideHotGrid)) : 0;
       if (overlap) {

@@ -332,8 +332,8 @@ int eps_hip_fill_u32(uint32_t* target, uint32_t value, uint64_t count, void* str
  * the push's stream and a side stream the library creates per thread and
  * device, forked after the gradient scan and joined before the checked apply;
  * the side stream takes the row kernels when some table of the push has
- * 65,536 or more references, or a sixteenth of the push's (its hot rows
- * outlast them), else the hot-row kernel.  Disabled: both on the push's stream, hot rows first (as
+ * 65,536 or more references (its hot rows outlast them), else the hot-row
+ * kernel.  Disabled: both on the push's stream, hot rows first (as
  * eps_hip_push_static does).  A push whose tables each take 128 or fewer
  * references has no hot rows and uses no side stream.  No counterpart in the
  * reference.  The side stream pays off when it has a hardware queue of its
