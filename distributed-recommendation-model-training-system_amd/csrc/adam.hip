@@ -671,10 +671,13 @@ struct FusedArgs {
   Control* ctrl;
   Bounds* bounds;
   GuardScalars gs;
-  uint32_t row_bits, cls, cls_end, vblocks, role, tables, features;  // classes [cls, cls_end)
-  uint32_t n;  // occurrences of the push (sorted positions, occurrence indices)
+  uint32_t row_bits, cls, cls_end, role, tables, features;  // classes [cls, cls_end)
+  uint32_t n;     // occurrences of the push (sorted positions, occurrence indices)
   uint32_t wide;  // every gradient array is 16-byte aligned: rows of dim % 4 == 0 too
-  uint32_t class_block[kClasses + 1];  // SortedReduceKernel: first block of each class (and the total)
+  // The short rows' windows: log2 of their positions per class, and each
+  // class's first block (and the total).  The long rows': log2 of theirs, and
+  // their units of kBlock columns at most.
+  uint32_t window_bits[kClasses], class_block[kClasses + 1], long_bits, long_slices;
 };
 static_assert(sizeof(FusedArgs) <= 4096, "update arguments fit the kernel-argument segment");
 
@@ -684,82 +687,107 @@ struct SortedShared {
   uint64_t rows[EPS_HIP_MAX_FEATURES];  // gradient rows per feature
   uint32_t heads[kBlock];
   uint32_t wave_heads[kBlock / kWave];
-  uint32_t mode, bad;
+  uint32_t mode;
+};
+struct LongRowShared {
+  uint32_t heads[kBlock], count[3], bad;
   RowSumShared sum;
 };
+__device__ __forceinline__ void StageSorted(const FusedArgs& a, SortedShared& sh) {
+  CopyWords(sh.t, a.t, sizeof(a.t));
+  CopyWords(sh.grad, a.grad, sizeof(a.grad));
+  CopyWords(sh.rows, a.grad_rows, sizeof(a.grad_rows));
+}
 
-// The rows whose first position lies in the windows of `ppb` positions that
-// virtual blocks vb, vb + step, ... < vblocks of the positions [start, end)
-// own.  A row of up to kBlockRowRefs references takes one group of 2^log2g
-// lanes (kGeneric: a wavefront over scalar columns), a longer one the block.
+// The row that starts at sorted position `sb`.  A key or reference naming
+// nothing of the push (a damaged workspace) is not used as an address: its
+// loads read zero and the row is not written.  The reference checks see the
+// same words in every lane.
+struct SortedRow { KeyParts kp; bool ok; uint64_t u; };
+template <bool kReduce>
+__device__ __forceinline__ SortedRow RowAt(const FusedArgs& a, const SortedShared& sh, uint32_t sb) {
+  SortedRow r;
+  r.kp = SplitKey(a.keys[sb], a.row_bits);
+  r.ok = KeyInRange(r.kp, a.tables, sh.t[min(r.kp.table, a.tables - 1)].rows);
+  r.u = 0;
+  if (kReduce) {
+    const uint32_t occ = a.vals[sb];
+    r.ok = r.ok && occ < a.n;
+    r.u = r.ok ? a.occ2u[occ] : 0;
+  }
+  return r;
+}
+
+// The rows of up to kBlockRowRefs references whose first position lies in the
+// windows of 2^window_bits positions that blocks vb, vb + step, ... of the
+// positions [start, end) own: a group of 2^log2g lanes a row (kGeneric: a
+// wavefront over scalar columns).  Only references of the row are loaded: a
+// batch filled up with repeats of the last one cost rows of one reference up
+// to twice their time (200,000 of dim 300 reduced, 306 -> 555 us).
 template <bool kGeneric, bool kReduce>
-__device__ __forceinline__ void SortedRows(const FusedArgs& a, SortedShared& sh, uint32_t start, uint32_t end,
-                                           uint32_t log2g, uint32_t ppb, uint32_t vb, uint32_t step,
-                                           uint32_t vblocks, bool write, RowStats& st) {
+__device__ __forceinline__ void ShortRows(const FusedArgs& a, SortedShared& sh, uint32_t start, uint32_t end,
+                                          uint32_t log2g, uint32_t window_bits, uint32_t vb, uint32_t step, bool write,
+                                          RowStats& st) {
   const uint32_t G = kGeneric ? kWave : (1u << log2g);
   const uint32_t lig = threadIdx.x & (G - 1);
   const uint32_t gid = threadIdx.x / G, ngroups = kBlock / G;
   const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const float* safe = reinterpret_cast<const float*>(a.ctrl);
-  for (; vb < vblocks; vb += step) {
-    const uint32_t p0 = start + vb * ppb;
-    if (p0 >= end) break;  // uniform: later virtual blocks are further right
-    const uint32_t p1 = min(p0 + ppb, end);
-    // Head positions of this block's range, in order.
+  const uint32_t window = 1u << window_bits, windows = (end - start + window - 1) >> window_bits;
+  for (; vb < windows; vb += step) {
+    const uint32_t p0 = start + (vb << window_bits);
+    const uint32_t p1 = min(p0 + window, end);
+    // Head positions of this window, in order.
     const uint32_t p = p0 + threadIdx.x;
-    const bool head = threadIdx.x < ppb && p < p1 && (p == start || a.keys[p] != a.keys[p - 1]);
+    const bool head = threadIdx.x < window && p < p1 && (p == start || a.keys[p] != a.keys[p - 1]);
     const uint64_t ballot = __ballot(head);
     if (lane == 0) sh.wave_heads[wave] = uint32_t(__popcll(ballot));
-    if (threadIdx.x == 0) sh.bad = 0;
     __syncthreads();
     uint32_t before = 0;
     for (uint32_t w = 0; w < wave; ++w) before += sh.wave_heads[w];
     const uint32_t nheads = sh.wave_heads[0] + sh.wave_heads[1] + sh.wave_heads[2] + sh.wave_heads[3];
     if (head) sh.heads[before + uint32_t(__popcll(ballot & ((1ull << lane) - 1)))] = p;
     __syncthreads();
-    if (!nheads) continue;
-    const uint32_t last_end = SegmentEndSearch(a.keys, p1, end, a.keys[p1 - 1]);
-    // What row h is: a key or reference naming nothing of the push (a damaged
-    // workspace) is not used as an address: its loads read zero and the row is
-    // not written.  The reference checks see the same words in every lane.
-    struct Row { uint32_t sb, se; KeyParts kp; bool ok; uint64_t u; };
-    auto row_of = [&](uint32_t h) {
-      Row r;
-      r.sb = sh.heads[h];
-      r.se = h + 1 < nheads ? sh.heads[h + 1] : last_end;
-      r.kp = SplitKey(a.keys[r.sb], a.row_bits);
-      r.ok = KeyInRange(r.kp, a.tables, sh.t[min(r.kp.table, a.tables - 1)].rows);
-      r.u = 0;
-      if (kReduce) {
-        const uint32_t occ = a.vals[r.sb];
-        r.ok = r.ok && occ < a.n;
-        r.u = r.ok ? a.occ2u[occ] : 0;
-      }
-      return r;
-    };
     for (uint32_t h = gid; h < nheads; h += ngroups) {
-      const Row row = row_of(h);
-      if (row.se - row.sb > kBlockRowRefs) continue;
+      const uint32_t sb = sh.heads[h];
+      uint32_t se;
+      if (h + 1 < nheads) {
+        se = sh.heads[h + 1];
+      } else {  // the window's last row: it may go on past the window
+        const uint32_t key = a.keys[sb];
+        if (sb + kBlockRowRefs < end && a.keys[sb + kBlockRowRefs] == key) continue;
+        se = SegmentEndSearch(a.keys, p1, min(end, sb + kBlockRowRefs), key);
+      }
+      const uint32_t cnt = se - sb;
+      if (cnt > kBlockRowRefs) continue;  // (LongRows)
+      const SortedRow row = RowAt<kReduce>(a, sh, sb);
       const TableDesc& T = sh.t[min(row.kp.table, a.tables - 1)];
-      bool ok = row.ok;
-      const uint32_t dim = T.dim, sb = row.sb, cnt = row.se - row.sb;
+      const uint32_t dim = T.dim;
       const SortedRefs refs{a.rs + sb, sh.grad, sh.rows, safe, a.features, dim};
+      bool ok = row.ok;
       if (!kGeneric) {
         const uint32_t c = lig * 4;
         const bool active = c < dim;
-        const uint32_t cl = active ? c : 0;
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (uint32_t k = 0; k < cnt; k += 4) {
-          float4 x[4];
-          float s[4];
-          uint64_t w[4];
+        for (uint32_t base = 0; base < cnt; base += G) {
+          const uint32_t here = min(G, cnt - base);
+          const uint64_t my = lig < here ? refs.Load(base + lig) : 0ull;
+          for (uint32_t k = 0; k < here; k += 4) {
+            float4 x[4];
+            float s[4];
 #pragma unroll
-          for (uint32_t q = 0; q < 4; ++q) w[q] = refs.Load(min(k + q, cnt - 1));
+            for (uint32_t q = 0; q < 4; ++q) {
+              const uint64_t w = __shfl(my, int(k + q), int(G));
+              bool in = true;
+              const float* src = refs.Source(w, active ? c : 0u, s[q], in);
+              const bool mine = k + q < here;
+              if (mine && !in) ok = false;
+              x[q] = mine && active ? Load4(src) : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
 #pragma unroll
-          for (uint32_t q = 0; q < 4; ++q) x[q] = Load4(refs.Source(w[q], cl, s[q], ok));
-#pragma unroll
-          for (uint32_t q = 0; q < 4; ++q)
-            if (k + q < cnt) Accumulate4(acc, x[q], s[q]);
+            for (uint32_t q = 0; q < 4; ++q)
+              if (k + q < here) Accumulate4(acc, x[q], s[q]);
+          }
         }
         if (!ok) st.err |= EPS_HIP_STATUS_BAD_INDEX;
         if (!active || !ok) continue;
@@ -771,24 +799,37 @@ __device__ __forceinline__ void SortedRows(const FusedArgs& a, SortedShared& sh,
           AdamRow4(T, row.kp.slot, c, acc, write, st);
         }
       } else {
-        for (uint32_t c0 = 0; c0 < dim; c0 += kWave) {
-          const uint32_t c = c0 + lig;
-          const bool active = c < dim;
-          const uint32_t cl = active ? c : c0;
+        // Lane l decodes reference l; the others take it from there.
+        static_assert(kBlockRowRefs <= kWave, "a reference a lane");
+        const uint32_t count = __builtin_amdgcn_readfirstlane(cnt);
+        float scale = 0.f;
+        bool in = true;
+        uint64_t src = 0;
+        if (lane < count) src = reinterpret_cast<uint64_t>(refs.Source(refs.Load(lane), 0, scale, in));
+        if (__ballot(!in)) ok = false;
+        auto source = [&](uint32_t k) {
+          const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(src), k);
+          const uint32_t hi = __builtin_amdgcn_readlane(uint32_t(src >> 32), k);
+          return reinterpret_cast<const float*>(lo | (uint64_t(hi) << 32));
+        };
+        auto scale_of = [&](uint32_t k) {
+          return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(scale), k));
+        };
+        if (!ok) {
+          st.err |= EPS_HIP_STATUS_BAD_INDEX;
+          continue;
+        }
+        for (uint32_t c = lane; c < dim; c += kWave) {
           float acc = 0.f;
-          for (uint32_t k = 0; k < cnt; k += 8) {
-            float x[8], s[8];
-            uint64_t w[8];
+          uint32_t k = 0;
+          for (; k + 4 <= count; k += 4) {
+            float x[4];
 #pragma unroll
-            for (uint32_t q = 0; q < 8; ++q) w[q] = refs.Load(min(k + q, cnt - 1));
+            for (uint32_t q = 0; q < 4; ++q) x[q] = LoadF(source(k + q) + c);
 #pragma unroll
-            for (uint32_t q = 0; q < 8; ++q) x[q] = LoadF(refs.Source(w[q], cl, s[q], ok));
-#pragma unroll
-            for (uint32_t q = 0; q < 8; ++q)
-              if (k + q < cnt) acc = acc + x[q] * s[q];
+            for (uint32_t q = 0; q < 4; ++q) acc = acc + x[q] * scale_of(k + q);
           }
-          if (!ok) st.err |= EPS_HIP_STATUS_BAD_INDEX;
-          if (!active || !ok) continue;
+          for (; k < count; ++k) acc = acc + LoadF(source(k) + c) * scale_of(k);
           if (kReduce) {
             if (!Finite(acc)) st.err |= EPS_HIP_STATUS_REDUCE_OVERFLOW;
             a.reduce_out[row.u * a.reduce_stride + c] = acc;
@@ -798,84 +839,154 @@ __device__ __forceinline__ void SortedRows(const FusedArgs& a, SortedShared& sh,
         }
       }
     }
-    // The window's long rows, one after another.
-    for (uint32_t h = 0; h < nheads; ++h) {
-      if ((h + 1 < nheads ? sh.heads[h + 1] : last_end) - sh.heads[h] <= kBlockRowRefs) continue;
-      const Row row = row_of(h);
-      const TableDesc& T = sh.t[min(row.kp.table, a.tables - 1)];
-      const SortedRefs refs{a.rs + row.sb, sh.grad, sh.rows, safe, a.features, T.dim};
-      for (uint32_t c0 = 0; c0 < T.dim; c0 += kBlock) {
-        bool ok = row.ok;
-        const bool wide = !kGeneric || (a.wide && T.dim % 4 == 0);  // uniform
-        const float acc = wide ? BlockRowSum<true>(sh.sum, refs, row.se - row.sb, T.dim, c0, 0.f, ok)
-                               : BlockRowSum<false>(sh.sum, refs, row.se - row.sb, T.dim, c0, 0.f, ok);
-        if (!ok) sh.bad = 1;
-        __syncthreads();
-        ok = sh.bad == 0;
-        __syncthreads();
-        if (threadIdx.x == 0) sh.bad = 0;
-        if (!ok) st.err |= EPS_HIP_STATUS_BAD_INDEX;
-        const uint32_t c = c0 + threadIdx.x;
-        if (c >= T.dim || !ok) continue;
-        if (kReduce) {
-          if (!Finite(acc)) st.err |= EPS_HIP_STATUS_REDUCE_OVERFLOW;
-          a.reduce_out[row.u * a.reduce_stride + c] = acc;
-        } else {
-          AdamRow1(T, row.kp.slot, c, acc, write, st);
-        }
-      }
-    }
     __syncthreads();
   }
 }
 
-__device__ __forceinline__ void StageSorted(const FusedArgs& a, SortedShared& sh) {
-  CopyWords(sh.t, a.t, sizeof(a.t));
-  CopyWords(sh.grad, a.grad, sizeof(a.grad));
-  CopyWords(sh.rows, a.grad_rows, sizeof(a.grad_rows));
+// The rows of more than kBlockRowRefs references whose first position lies in
+// the windows of 2^long_bits positions (at most kBlock) that blocks vb, vb +
+// step, ... of the positions [start, end) own, one after another, each by the
+// whole block.  A row of more than kBlock columns is that many units, of kBlock
+// columns each, on different blocks.  False when there is none: nothing was
+// staged then.
+template <bool kReduce>
+__device__ __forceinline__ bool LongRows(const FusedArgs& a, SortedShared& sh, LongRowShared& lsh, bool staged,
+                                         uint32_t start, uint32_t end, uint32_t vb, uint32_t step, bool write,
+                                         RowStats& st) {
+  const float* safe = reinterpret_cast<const float*>(a.ctrl);
+  const uint32_t window = 1u << a.long_bits, windows = (end - start + window - 1) >> a.long_bits;
+  bool found = false;
+  if (threadIdx.x == 0) lsh.count[0] = lsh.bad = 0;
+  __syncthreads();
+  // (The counts go round three words, so that no thread still reads the one
+  // that another clears.)
+  for (uint32_t i = 0; vb < windows * a.long_slices; vb += step, i = i == 2 ? 0 : i + 1) {
+    const uint32_t slice = vb / windows, c0 = slice * kBlock;
+    const uint32_t p = start + ((vb - slice * windows) << a.long_bits) + threadIdx.x;
+    if (threadIdx.x < window && p + kBlockRowRefs < end) {
+      const uint32_t key = a.keys[p], ahead = a.keys[p + kBlockRowRefs], before = p == start ? ~key : a.keys[p - 1];
+      if (key == ahead && key != before) lsh.heads[atomicAdd(&lsh.count[i], 1u)] = p;
+    }
+    if (threadIdx.x == 0) lsh.count[i == 2 ? 0 : i + 1] = 0;
+    __syncthreads();
+    const uint32_t rows = lsh.count[i];
+    if (rows && !found && !staged) {
+      StageSorted(a, sh);
+      __syncthreads();
+    }
+    found = found || rows;
+    for (uint32_t h = 0; h < rows; ++h) {
+      const uint32_t sb = lsh.heads[h], se = SegmentEndSearch(a.keys, sb + kBlockRowRefs + 1, end, a.keys[sb]);
+      const SortedRow row = RowAt<kReduce>(a, sh, sb);
+      const TableDesc& T = sh.t[min(row.kp.table, a.tables - 1)];
+      const SortedRefs refs{a.rs + sb, sh.grad, sh.rows, safe, a.features, T.dim};
+      if (c0 >= T.dim) continue;  // uniform
+      // (Vector classes load 16 bytes wherever their gradients lie, as their own kernels do.)
+      bool ok = row.ok;
+      const float acc = T.dim % 4 == 0 && (T.dim <= 256 || a.wide)
+                            ? BlockRowSum<true>(lsh.sum, refs, se - sb, T.dim, c0, 0.f, ok)
+                            : BlockRowSum<false>(lsh.sum, refs, se - sb, T.dim, c0, 0.f, ok);
+      if (!ok) lsh.bad = 1;
+      __syncthreads();
+      ok = lsh.bad == 0;
+      __syncthreads();
+      if (threadIdx.x == 0) lsh.bad = 0;
+      if (!ok) st.err |= EPS_HIP_STATUS_BAD_INDEX;
+      const uint32_t c = c0 + threadIdx.x;
+      if (c >= T.dim || !ok) continue;
+      if (kReduce) {
+        if (!Finite(acc)) st.err |= EPS_HIP_STATUS_REDUCE_OVERFLOW;
+        a.reduce_out[row.u * a.reduce_stride + c] = acc;
+      } else {
+        AdamRow1(T, row.kp.slot, c, acc, write, st);
+      }
+    }
+  }
+  return found;
 }
+
+// The sorted positions of classes [first, last), from the workspace, kept
+// inside the push's.
+__device__ __forceinline__ uint2 ClassRange(const FusedArgs& a, uint32_t first, uint32_t last) {
+  const uint32_t begin = a.ctrl->class_start[first], stop = a.ctrl->class_start[last];
+  const uint32_t end = min(stop, a.n);
+  return make_uint2(min(begin, end), end);
+}
+
+// Which rows a launch of the sorted driver takes.  Long rows need 40 KB of LDS
+// and about 140 registers, three blocks a CU; rows of a few references are a
+// chain of memory latencies, and want more of them.  So the rows of more than
+// kBothBlocks windows, whose blocks would wait for room, are taken by two
+// launches: 43,000 uniform references on each of 26 tables of dim 64 reduced,
+// 422 us with both in one, 275 apart; 200,000 of dim 300 pushed, 909 and 425
+// (20,000 of dim 50, 2,500 windows, 33 and 28).  Fewer take one, and save a
+// launch: 400 or 4,000 references of dim 50, 15 us and 18 apart.  The two do
+// not overlap, which costs skewed ids what the long rows took beside the short
+// ones (43,000 of dim 10, Zipf of 1.05, 75 -> 87).
+enum SortedPart : uint32_t { kShortPart = 1, kLongPart = 2, kBothParts = 3 };
 
 // Adam of the generic class (one wavefront per row, scalar columns), and the
 // checked apply of every class.
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) SortedUpdateKernel(FusedArgs a) {
+template <uint32_t kPart>
+__device__ __forceinline__ void SortedUpdate(const FusedArgs& a) {
   // The checked apply nearly always has nothing to do.
   if (a.role == kFallback && a.ctrl->mode != kChecked) return;
   __shared__ SortedShared sh;
   Control* ctrl = a.ctrl;
   const GuardInputs in = LoadGuard(ctrl);
-  StageSorted(a, sh);
+  if (kPart & kShortPart) StageSorted(a, sh);
   bool write = true;
   if (!LaunchGate(ctrl, in, sh.t, a.gs, a.role, &sh.mode, write)) return;
-  // The classes' sorted positions, from the workspace, kept inside the push's.
-  const uint32_t first = ctrl->class_start[a.cls], last = ctrl->class_start[a.cls_end];
-  const uint32_t end = min(last, a.n), start = min(first, end);
+  const uint2 range = ClassRange(a, a.cls, a.cls_end);
   RowStats st;
   __syncthreads();
-  SortedRows<true, false>(a, sh, start, end, 6, PositionsPerBlock(kClasses - 1), blockIdx.x, gridDim.x, a.vblocks,
-                          write, st);
+  if constexpr (kPart & kShortPart)
+    ShortRows<true, false>(a, sh, range.x, range.y, 6, a.window_bits[kClasses - 1], blockIdx.x, gridDim.x, write, st);
+  if constexpr (kPart & kLongPart) {
+    __shared__ LongRowShared lsh;
+    const bool found = LongRows<false>(a, sh, lsh, kPart & kShortPart, range.x, range.y, blockIdx.x, gridDim.x, write,
+                                       st);
+    if (!found && !(kPart & kShortPart)) return;
+  }
   FinishBlock(st, ctrl, a.bounds, write);
 }
+__global__ void __launch_bounds__(kBlock) SortedUpdateKernel(FusedArgs a) { SortedUpdate<kShortPart>(a); }
+__global__ void __launch_bounds__(kBlock) LongUpdateKernel(FusedArgs a) { SortedUpdate<kLongPart>(a); }
+__global__ void __launch_bounds__(kBlock) SortedLongUpdateKernel(FusedArgs a) { SortedUpdate<kBothParts>(a); }
 
-// Reduced gradients of every class in one launch (class c has the blocks
-// [class_block[c], class_block[c + 1])): the classes' long rows then overlap.
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) SortedReduceKernel(FusedArgs a) {
+// Reduced gradients of every class in one launch: the short rows of class c
+// have the blocks [class_block[c], class_block[c + 1]), the long rows of every
+// class all of them.
+template <uint32_t kPart>
+__device__ __forceinline__ void SortedReduce(const FusedArgs& a) {
   __shared__ SortedShared sh;
-  StageSorted(a, sh);
   Control* ctrl = a.ctrl;
-  uint32_t cls = 0;
-#pragma unroll
-  for (uint32_t c = 1; c < kClasses; ++c) cls += blockIdx.x >= a.class_block[c];
-  const uint32_t first = ctrl->class_start[cls], last = ctrl->class_start[cls + 1];
-  const uint32_t end = min(last, a.n), start = min(first, end);
-  const uint32_t block = blockIdx.x - a.class_block[cls];
   RowStats st;
-  __syncthreads();
-  if (cls + 1 == kClasses)
-    SortedRows<true, true>(a, sh, start, end, 6, PositionsPerBlock(cls), block, block + 1, block + 1, false, st);
-  else
-    SortedRows<false, true>(a, sh, start, end, cls + 2, PositionsPerBlock(cls), block, block + 1, block + 1, false, st);
+  if constexpr (kPart & kShortPart) {
+    StageSorted(a, sh);
+    uint32_t cls = 0;
+#pragma unroll
+    for (uint32_t c = 1; c < kClasses; ++c) cls += blockIdx.x >= a.class_block[c];
+    const uint2 range = ClassRange(a, cls, cls + 1);
+    const uint32_t block = blockIdx.x - a.class_block[cls], grid = a.class_block[cls + 1] - a.class_block[cls];
+    __syncthreads();
+    if (cls + 1 == kClasses)
+      ShortRows<true, true>(a, sh, range.x, range.y, 6, a.window_bits[cls], block, grid, false, st);
+    else
+      ShortRows<false, true>(a, sh, range.x, range.y, cls + 2, a.window_bits[cls], block, grid, false, st);
+  }
+  if constexpr (kPart & kLongPart) {
+    __shared__ LongRowShared lsh;
+    const uint2 range = ClassRange(a, 0, kClasses);
+    const bool found = LongRows<true>(a, sh, lsh, kPart & kShortPart, range.x, range.y, blockIdx.x, gridDim.x, false,
+                                      st);
+    if (!found && !(kPart & kShortPart)) return;
+  }
   FinishBlock(st, ctrl, nullptr, false);
 }
+__global__ void __launch_bounds__(kBlock) SortedReduceKernel(FusedArgs a) { SortedReduce<kShortPart>(a); }
+__global__ void __launch_bounds__(kBlock) LongReduceKernel(FusedArgs a) { SortedReduce<kLongPart>(a); }
+__global__ void __launch_bounds__(kBlock) SortedLongReduceKernel(FusedArgs a) { SortedReduce<kBothParts>(a); }
 
 // ---------------------------------------------------------------------------
 // Vector-class update (dim % 4 == 0, dim <= 256).  Two kernels:
@@ -2267,6 +2378,9 @@ constexpr int kPrimary = 1, kSecond = 2, kOneStream = 4, kForked = 8;
 constexpr uint64_t kVectorGrid = 4096;  // persistent grid cap of the vector kernels
 constexpr uint64_t kSecondGrid = 32;      // grid cap of the checked apply: it usually exits at
                                           // once, and a small grid launches faster
+constexpr uint32_t kApplyWindowBits = 5;  // its windows of sorted positions
+constexpr uint64_t kBothBlocks = 1024;    // windows up to which one launch takes short and long rows
+constexpr uint64_t kLongGrid = 2048;      // grid cap of the long rows' launches
 constexpr uint64_t kHotGrid = 512;      // two blocks per CU (LDS: four 17 KiB tiles per block)
 // Blocks of the 64-column hot-row kernel beside the row kernels: enough to
 // finish the hot rows well before the row kernels do, few enough to leave
@@ -2511,6 +2625,28 @@ int RunSorted(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, 
       if (overlap && !joined) EPS_HIP_TRY(Check(hipEventRecord(ov->join, ov->side), "update join"));
     }
   }
+  // The sorted driver's launches.  Whether a table of classes [first, kClasses)
+  // has references enough for a long row:
+  auto may_be_long = [&](uint32_t first) {
+    uint64_t refs[EPS_HIP_MAX_TABLES] = {};
+    for (uint32_t f = 0; f < feature_count; ++f) refs[features[f].table] += features[f].occurrences;
+    for (uint32_t t = 0; t < table_count; ++t)
+      if (DimClass(tables[t].dim) >= first && refs[t] > kBlockRowRefs) return true;
+    return false;
+  };
+  for (uint32_t cls = 0; cls < kClasses; ++cls) {
+    a.window_bits[cls] = 0;
+    while ((2u << a.window_bits[cls]) <= PositionsPerBlock(cls)) ++a.window_bits[cls];
+  }
+  // Long rows' windows: as many positions as threads to look at them, fewer
+  // where that leaves blocks idle.
+  a.long_slices = 1;
+  for (uint32_t t = 0; t < table_count; ++t)
+    a.long_slices = std::max(a.long_slices, (tables[t].dim + kBlock - 1) / kBlock);
+  auto long_grid = [&](uint64_t positions) {
+    a.long_bits = positions >= (kLongGrid << 8) ? 8 : 6;
+    return unsigned(std::min<uint64_t>(((positions + (1u << a.long_bits) - 1) >> a.long_bits) * a.long_slices, kLongGrid));
+  };
   if (reduce) {
     uint64_t blocks = 0;
     for (uint32_t cls = 0; cls < kClasses; ++cls) {
@@ -2518,32 +2654,50 @@ int RunSorted(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, 
       blocks += (plan.class_occurrences[cls] + PositionsPerBlock(cls) - 1) / PositionsPerBlock(cls);
     }
     a.class_block[kClasses] = uint32_t(blocks);
-    hipLaunchKernelGGL(SortedReduceKernel, dim3(unsigned(blocks)), dim3(kBlock), 0, s, a);
+    const unsigned grid = long_grid(plan.occurrences);
+    const bool apart = blocks > kBothBlocks;
+    if (!may_be_long(0) || apart)
+      hipLaunchKernelGGL(SortedReduceKernel, dim3(unsigned(blocks)), dim3(kBlock), 0, s, a);
+    else
+      hipLaunchKernelGGL(SortedLongReduceKernel, dim3(unsigned(blocks)), dim3(kBlock), 0, s, a);
     EPS_HIP_LAUNCHED("sorted reduce");
+    if (may_be_long(0) && apart) {
+      hipLaunchKernelGGL(LongReduceKernel, dim3(grid), dim3(kBlock), 0, s, a);
+      EPS_HIP_LAUNCHED("sorted reduce (long rows)");
+    }
     return EPS_HIP_OK;
   }
   // The generic class.
   if ((phases & kPrimary) && plan.class_occurrences[kClasses - 1]) {
-    const uint32_t ppb = PositionsPerBlock(kClasses - 1);
+    const uint64_t positions = plan.class_occurrences[kClasses - 1];
+    const uint64_t blocks = (positions + PositionsPerBlock(kClasses - 1) - 1) / PositionsPerBlock(kClasses - 1);
     a.cls = kClasses - 1;
     a.cls_end = kClasses;
-    a.vblocks = uint32_t((plan.class_occurrences[kClasses - 1] + ppb - 1) / ppb);
     a.role = role;
-    hipLaunchKernelGGL(SortedUpdateKernel, dim3(a.vblocks), dim3(kBlock), 0, s, a);
+    const unsigned grid = long_grid(positions);
+    const bool apart = blocks > kBothBlocks, any_long = may_be_long(kClasses - 1);
+    auto kernel = any_long && !apart ? SortedLongUpdateKernel : SortedUpdateKernel;
+    hipLaunchKernelGGL(kernel, dim3(unsigned(blocks)), dim3(kBlock), 0, s, a);
     EPS_HIP_LAUNCHED("sorted update");
+    if (any_long && apart) {
+      a.role = kFollow;
+      hipLaunchKernelGGL(LongUpdateKernel, dim3(grid), dim3(kBlock), 0, s, a);
+      EPS_HIP_LAUNCHED("sorted update (long rows)");
+    }
   }
   if (overlap && (phases & kPrimary)) EPS_HIP_TRY(Check(hipStreamWaitEvent(s, ov->join, 0), "hot-row join wait"));
   // The checked apply (after a validate-only pass) is one launch over every
   // class, one wavefront per row: it usually exits at once, and when it runs
   // it adds each row's references in the same order as the passes above.
   if (phases & kSecond) {
-    const uint32_t ppb = PositionsPerBlock(kClasses - 1);
     a.cls = 0;
     a.cls_end = kClasses;
-    a.vblocks = uint32_t((plan.occurrences + ppb - 1) / ppb);
     a.role = kFallback;
-    if (a.vblocks) {
-      hipLaunchKernelGGL(SortedUpdateKernel, dim3(std::min<uint32_t>(a.vblocks, kSecondGrid)),
+    a.window_bits[kClasses - 1] = kApplyWindowBits;
+    a.long_bits = 8;
+    const uint64_t windows = (plan.occurrences + (1u << kApplyWindowBits) - 1) >> kApplyWindowBits;
+    if (windows) {
+      hipLaunchKernelGGL(SortedLongUpdateKernel, dim3(unsigned(std::min<uint64_t>(windows, kSecondGrid))),
                          dim3(kBlock), 0, s, a);
       EPS_HIP_LAUNCHED("sorted update (checked apply)");
     }

@@ -13,8 +13,19 @@ pytestmark = pytest.mark.gpu
 F32 = np.float32
 
 
-def lengths_of(dim):
-    """Row lengths around the hand-over to the block and its tiles."""
+def block_lengths(dim):
+    """Row lengths around the hand-over to the block, its tiles (4,096 products of 16-byte loads, 2,048 of scalar
+    ones, a tile row the next power of two of the columns) and its groups of 128 references."""
+    pitch = 32 if dim % 4 == 0 else 16
+    while pitch < min(dim, 256):
+        pitch *= 2
+    tile = (4096 if dim % 4 == 0 else 2048) // pitch
+    edges = [tile - 1, tile, tile + 1, 2 * tile - 1, 2 * tile, 3 * tile + 1, 127, 128, 129, 255, 256, 257]
+    return [1, 2, 4, 5, 8, 9, 31, 32, 33, 48, 49] + sorted({max(e, 33) for e in edges})
+
+
+def csr_lengths(dim):
+    """Row lengths around the hand-over to the block of a CSR packet, and its tiles."""
     vector = dim % 4 == 0 and dim <= 256
     width = dim // 4 if vector else min(dim, 256)
     lanes = 4
@@ -40,7 +51,7 @@ def feature_of(W, rng, dim, lengths, rows):
 def test_reduce_long_rows(torch_gpu, pkg, dim):
     torch, W, H = torch_gpu, pkg.workloads, pkg.eps_hip
     rng = np.random.default_rng(dim)
-    lengths = lengths_of(dim)
+    lengths = block_lengths(dim)
     specs = [W.TableSpec(0, dim, 400, seed=3)]
     feats = [feature_of(W, rng, dim, lengths, specs[0].rows)]
     print(f"case: dim={dim} row lengths {lengths}", flush=True)
@@ -52,7 +63,7 @@ def test_push_long_generic_rows(torch_gpu, pkg, dim):
     torch, W, H = torch_gpu, pkg.workloads, pkg.eps_hip
     rng = np.random.default_rng(1000 + dim)
     spec = W.TableSpec(0, dim, 400, seed=4)
-    f = feature_of(W, rng, dim, lengths_of(dim), spec.rows)
+    f = feature_of(W, rng, dim, block_lengths(dim), spec.rows)
     print(f"case: dim={dim} occurrences={len(f.keys)}", flush=True)
     shard = H.DeviceShard(torch, [spec])
     shard.init_rows()
@@ -68,13 +79,85 @@ def test_push_long_generic_rows(torch_gpu, pkg, dim):
     assert_close(got.reshape(want.shape), want, f"generic push dim={dim}", strict_ulp=0)
 
 
+def crowded_lengths(rng, dim, short):
+    """The edges among `short` rows of 1 to 6 references: more than 1,024 windows of 8 positions."""
+    return list(rng.permutation(np.concatenate([block_lengths(dim), [1000], rng.integers(1, 7, short)])))
+
+
+# (520 and 514: rows of three units of columns, of 16-byte and scalar loads.)
+@pytest.mark.parametrize("dim", [3, 50, 300, 520, 514])
+def test_push_long_generic_rows_apart(torch_gpu, pkg, dim):
+    """A push of enough positions that its short and long rows are launched apart."""
+    torch, W, H = torch_gpu, pkg.workloads, pkg.eps_hip
+    rng = np.random.default_rng(5000 + dim)
+    spec = W.TableSpec(0, dim, 4000, seed=4)
+    f = feature_of(W, rng, dim, crowded_lengths(rng, dim, 3000), spec.rows)
+    assert len(f.keys) > 8 * 1024
+    print(f"case: dim={dim} occurrences={len(f.keys)}", flush=True)
+    shard = H.DeviceShard(torch, [spec])
+    shard.init_rows()
+    dev = [H.DeviceFeature(torch, f)]
+    shard.prepare(dev)
+    assert shard.push(dev) & H.STATUS_ERRORS == 0
+    store = oracle_store(spec)
+    store.prepare(f)
+    assert oracle.push([store], [f], [0], [f.gradient]) == 0
+    keys = store.keys()
+    want, _ = store.read_many(keys)
+    got = shard.read_rows(0, torch.from_numpy(keys.view(np.int64)).cuda()).cpu().numpy()
+    assert_close(got.reshape(want.shape), want, f"generic push dim={dim}", strict_ulp=0)
+
+
+def test_reduce_long_rows_apart(torch_gpu, pkg):
+    """Every class in one call, short and long rows apart, rows that end with their class among them."""
+    torch, W, H = torch_gpu, pkg.workloads, pkg.eps_hip
+    rng = np.random.default_rng(6000)
+    dims = [4, 300, 64, 10, 128, 256, 520, 32]
+    specs = [W.TableSpec(i, d, 1500, seed=3 + i) for i, d in enumerate(dims)]
+    feats = []
+    for i, d in enumerate(dims):
+        f = feature_of(W, rng, d, crowded_lengths(rng, d, 700), 1500)
+        f.keys[f.keys == f.keys.max()] = 1499  # the last slot
+        f.table = i
+        feats.append(f)
+    print(f"case: dims={dims} occurrences={sum(len(f.keys) for f in feats)}", flush=True)
+    check_unique_reduce(torch, W, H, specs, feats)
+
+
+@pytest.mark.parametrize("dims", [[300], [50, 64, 3]])
+def test_checked_apply_of_long_rows(torch_gpu, pkg, dims):
+    """The two-pass update (a bound the guard cannot prove safe) over short and long rows of vector and generic
+    classes leaves the state of the fused one."""
+    torch, W, H = torch_gpu, pkg.workloads, pkg.eps_hip
+    rng = np.random.default_rng(7000 + len(dims))
+    specs = [W.TableSpec(i, d, 4000, seed=5 + i) for i, d in enumerate(dims)]
+    feats = []
+    for i, d in enumerate(dims):
+        f = feature_of(W, rng, d, crowded_lengths(rng, d, 2500), 4000)
+        f.table = i
+        feats.append(f)
+    print(f"case: dims={dims} occurrences={sum(len(f.keys) for f in feats)}", flush=True)
+    states = []
+    for bound in (None, 2e30):
+        shard = H.DeviceShard(torch, specs)
+        shard.init_rows()
+        if bound:
+            shard.bounds.view(torch.float32)[0] = bound
+        dev = [H.DeviceFeature(torch, f) for f in feats]
+        shard.prepare(dev)
+        status = shard.push(dev)
+        assert status & H.STATUS_ERRORS == 0 and bool(status & H.STATUS_CHECKED_PATH) == bool(bound)
+        states.append([s.cpu().numpy() for s in shard.state])
+    assert all(np.array_equal(a, b) for a, b in zip(*states))
+
+
 @pytest.mark.parametrize("dim", [4, 64, 100, 256, 3, 50, 300])
 def test_compact_long_rows(torch_gpu, pkg, dim):
     torch, W, H = torch_gpu, pkg.workloads, pkg.eps_hip
     rng = np.random.default_rng(2000 + dim)
     spec = W.TableSpec(0, dim, 4000, seed=5)
     # An empty row, the edges, and enough short rows for several virtual blocks.
-    lengths = np.array([0] + lengths_of(dim) + list(rng.integers(0, 7, 700)))
+    lengths = np.array([0] + csr_lengths(dim) + list(rng.integers(0, 7, 700)))
     rows, count = len(lengths), 300
     slots = rng.permutation(spec.rows)[:rows]
     offsets = np.concatenate([[0], np.cumsum(lengths)]).astype(np.uint64)
@@ -103,7 +186,7 @@ def test_compact_long_rows(torch_gpu, pkg, dim):
 
 @pytest.mark.parametrize("dim", [4, 16, 64, 256, 6, 33, 260, 301])
 def test_reduce_rows_of_several_tiles(torch_gpu, pkg, dim):
-    """Rows of several tiles and groups of 256 references: the last one full, one short and one over."""
+    """Rows of several tiles and groups of 128 references: the last one full, one short and one over."""
     torch, W, H = torch_gpu, pkg.workloads, pkg.eps_hip
     rng = np.random.default_rng(3000 + dim)
     lengths = [33, 63, 64, 65, 127, 129, 255, 256, 257, 511, 513, 768, 769, 1025, 1281]
