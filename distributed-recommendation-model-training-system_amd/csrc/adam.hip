@@ -2381,6 +2381,9 @@ constexpr uint64_t kSecondGrid = 32;      // grid cap of the checked apply: it u
 constexpr uint32_t kApplyWindowBits = 5;  // its windows of sorted positions
 constexpr uint64_t kBothBlocks = 1024;    // windows up to which one launch takes short and long rows
 constexpr uint64_t kLongGrid = 2048;      // grid cap of the long rows' launches
+// Grid cap of a class's short rows: six classes in one launch stay below the
+// 2^32 threads that one can have.
+constexpr uint64_t kSortedGrid = 1ull << 21;
 constexpr uint64_t kHotGrid = 512;      // two blocks per CU (LDS: four 17 KiB tiles per block)
 // Blocks of the 64-column hot-row kernel beside the row kernels: enough to
 // finish the hot rows well before the row kernels do, few enough to leave
@@ -2651,7 +2654,8 @@ int RunSorted(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, 
     uint64_t blocks = 0;
     for (uint32_t cls = 0; cls < kClasses; ++cls) {
       a.class_block[cls] = uint32_t(blocks);
-      blocks += (plan.class_occurrences[cls] + PositionsPerBlock(cls) - 1) / PositionsPerBlock(cls);
+      blocks += std::min<uint64_t>((plan.class_occurrences[cls] + PositionsPerBlock(cls) - 1) / PositionsPerBlock(cls),
+                                   kSortedGrid);
     }
     a.class_block[kClasses] = uint32_t(blocks);
     const unsigned grid = long_grid(plan.occurrences);
@@ -2677,7 +2681,7 @@ int RunSorted(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, 
     const unsigned grid = long_grid(positions);
     const bool apart = blocks > kBothBlocks, any_long = may_be_long(kClasses - 1);
     auto kernel = any_long && !apart ? SortedLongUpdateKernel : SortedUpdateKernel;
-    hipLaunchKernelGGL(kernel, dim3(unsigned(blocks)), dim3(kBlock), 0, s, a);
+    hipLaunchKernelGGL(kernel, dim3(unsigned(std::min<uint64_t>(blocks, kSortedGrid))), dim3(kBlock), 0, s, a);
     EPS_HIP_LAUNCHED("sorted update");
     if (any_long && apart) {
       a.role = kFollow;
