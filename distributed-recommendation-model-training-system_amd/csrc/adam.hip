@@ -452,6 +452,11 @@ __device__ void FinishBlock(const RowStats& st, Control* ctrl, Bounds* bounds, b
 // those eight tables.
 constexpr uint32_t kBlockRowRefs = 32;   // rows with more references are summed by the block
 constexpr uint32_t kLongTile = 4096;     // floats of a staged tile (of two)
+// Columns of a row that one block sums; wider rows are units of as many, on
+// different blocks.  (43,000 references of dim 300, Zipf of 1.05, pushed: units
+// of 256 columns 273 us, of 128 163.  Of 64, 133, but a CSR packet of 200,000
+// references in rows of 65, dim 256, 110 instead of 76.)
+constexpr uint32_t kLongColumns = 128;
 
 // Waits for this wave's LDS accesses, then for the block's other waves: unlike
 // __syncthreads it leaves global loads in flight.
@@ -534,8 +539,8 @@ struct RowSumShared {
   float scale[2][kRefGroup];
 };
 
-// `acc` plus references [0, count) of column c0 + threadIdx.x (`acc` when that
-// lies past the dimension).  kVec: rows are 16-byte aligned and dim % 4 == 0.
+// `acc` plus references [0, count) of column c0 + threadIdx.x (`acc` past the
+// unit's columns).  kVec: rows are 16-byte aligned and dim % 4 == 0.
 // `ok` turns false in any thread that met a reference of no gradient row.
 // Called by the whole block.  A thread each decodes the references of a group
 // of 128 to LDS, a group ahead of the row loads, so that these wait for no
@@ -549,12 +554,12 @@ __device__ __forceinline__ float BlockRowSum(RowSumShared& sh, const Refs& refs,
   constexpr uint32_t kLoads = kTile / (kBlock * kCols);          // loads of a thread per tile
   constexpr uint32_t kDepth = 2;                                 // tiles of rows in flight
   constexpr uint32_t kAddRows = kVec ? 16 : 8;
-  static_assert(kTile / 256 % kAddRows == 0 && kTile / (kVec ? 32 : 16) <= kRefGroup, "tiles of whole steps, in a group");
+  static_assert(kTile / kLongColumns % kAddRows == 0 && kTile / (kVec ? 32 : 16) <= kRefGroup, "tiles of whole steps, in a group");
   static_assert(kDepth % 2 == 0, "a slot's tiles lie in one half of the LDS");
-  const uint32_t cols = min(dim - c0, kBlock);
+  const uint32_t cols = min(dim - c0, kLongColumns);
   uint32_t log2g = kVec ? 3 : 4;                                 // lanes of a reference
   while ((kCols << log2g) < cols) ++log2g;
-  const uint32_t pitch = kCols << log2g;                         // 16 to 256
+  const uint32_t pitch = kCols << log2g;                         // 16 to 128
   const uint32_t per_step = kBlock >> log2g, tile_refs = kTile / pitch;
   const uint32_t sub = threadIdx.x >> log2g, e = (threadIdx.x & ((1u << log2g) - 1)) * kCols;
   const uint32_t at = e < cols ? e : 0u;
@@ -641,8 +646,7 @@ __device__ __forceinline__ float BlockRowSum(RowSumShared& sh, const Refs& refs,
           case 16: acc = AddTile<16, kAddRows>(col, n, acc); break;
           case 32: acc = AddTile<32, kAddRows>(col, n, acc); break;
           case 64: acc = AddTile<64, kAddRows>(col, n, acc); break;
-          case 128: acc = AddTile<128, kAddRows>(col, n, acc); break;
-          default: acc = AddTile<256, kAddRows>(col, n, acc); break;
+          default: acc = AddTile<128, kAddRows>(col, n, acc); break;
         }
       }
       base += tile_refs;
@@ -676,7 +680,7 @@ struct FusedArgs {
   uint32_t wide;  // every gradient array is 16-byte aligned: rows of dim % 4 == 0 too
   // The short rows' windows: log2 of their positions per class, and each
   // class's first block (and the total).  The long rows': log2 of theirs, and
-  // their units of kBlock columns at most.
+  // the units of columns of the widest table's.
   uint32_t window_bits[kClasses], class_block[kClasses + 1], long_bits, long_slices;
 };
 static_assert(sizeof(FusedArgs) <= 4096, "update arguments fit the kernel-argument segment");
@@ -846,8 +850,7 @@ __device__ __forceinline__ void ShortRows(const FusedArgs& a, SortedShared& sh, 
 // The rows of more than kBlockRowRefs references whose first position lies in
 // the windows of 2^long_bits positions (at most kBlock) that blocks vb, vb +
 // step, ... of the positions [start, end) own, one after another, each by the
-// whole block.  A row of more than kBlock columns is that many units, of kBlock
-// columns each, on different blocks.  False when there is none: nothing was
+// whole block (a unit of its columns).  False when there is none: nothing was
 // staged then.
 template <bool kReduce>
 __device__ __forceinline__ bool LongRows(const FusedArgs& a, SortedShared& sh, LongRowShared& lsh, bool staged,
@@ -861,7 +864,7 @@ __device__ __forceinline__ bool LongRows(const FusedArgs& a, SortedShared& sh, L
   // (The counts go round three words, so that no thread still reads the one
   // that another clears.)
   for (uint32_t i = 0; vb < windows * a.long_slices; vb += step, i = i == 2 ? 0 : i + 1) {
-    const uint32_t slice = vb / windows, c0 = slice * kBlock;
+    const uint32_t slice = vb / windows, c0 = slice * kLongColumns;
     const uint32_t p = start + ((vb - slice * windows) << a.long_bits) + threadIdx.x;
     if (threadIdx.x < window && p + kBlockRowRefs < end) {
       const uint32_t key = a.keys[p], ahead = a.keys[p + kBlockRowRefs], before = p == start ? ~key : a.keys[p - 1];
@@ -893,7 +896,7 @@ __device__ __forceinline__ bool LongRows(const FusedArgs& a, SortedShared& sh, L
       if (threadIdx.x == 0) lsh.bad = 0;
       if (!ok) st.err |= EPS_HIP_STATUS_BAD_INDEX;
       const uint32_t c = c0 + threadIdx.x;
-      if (c >= T.dim || !ok) continue;
+      if (threadIdx.x >= kLongColumns || c >= T.dim || !ok) continue;
       if (kReduce) {
         if (!Finite(acc)) st.err |= EPS_HIP_STATUS_REDUCE_OVERFLOW;
         a.reduce_out[row.u * a.reduce_stride + c] = acc;
@@ -2645,7 +2648,7 @@ int RunSorted(const eps_hip_table* tables, const eps_hip_optimizer* optimizers, 
   // where that leaves blocks idle.
   a.long_slices = 1;
   for (uint32_t t = 0; t < table_count; ++t)
-    a.long_slices = std::max(a.long_slices, (tables[t].dim + kBlock - 1) / kBlock);
+    a.long_slices = std::max(a.long_slices, (tables[t].dim + kLongColumns - 1) / kLongColumns);
   auto long_grid = [&](uint64_t positions) {
     a.long_bits = positions >= (kLongGrid << 8) ? 8 : 6;
     return unsigned(std::min<uint64_t>(((positions + (1u << a.long_bits) - 1) >> a.long_bits) * a.long_slices, kLongGrid));

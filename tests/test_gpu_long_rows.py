@@ -17,7 +17,7 @@ def block_lengths(dim):
     """Row lengths around the hand-over to the block, its tiles (4,096 products of 16-byte loads, 2,048 of scalar
     ones, a tile row the next power of two of the columns) and its groups of 128 references."""
     pitch = 32 if dim % 4 == 0 else 16
-    while pitch < min(dim, 256):
+    while pitch < min(dim, 128):
         pitch *= 2
     tile = (4096 if dim % 4 == 0 else 2048) // pitch
     edges = [tile - 1, tile, tile + 1, 2 * tile - 1, 2 * tile, 3 * tile + 1, 127, 128, 129, 255, 256, 257]
