@@ -40,6 +40,11 @@ namespace eps_hip {
 namespace {
 
 constexpr uint32_t kFallbackGrid = 2048;
+// Blocks of a CSR packet's tail, which has nothing to do for many packets (2,000
+// rows without a long one: 512 blocks 15.0 us a call, 1,024 15.8); packets of
+// kTailRows rows and more take twice as many.
+constexpr uint32_t kTailGrid = 512;
+constexpr uint64_t kTailRows = 1ull << 15;
 
 // ---------------------------------------------------------------------------
 // Gradient scan (GradMaxKernel), the first kernel of an update.  Its spans are
@@ -2054,7 +2059,7 @@ struct RowArgs {
   Control* ctrl;
   Bounds* bounds;
   GuardScalars gs;
-  uint32_t log2g, vblocks, role;
+  uint32_t log2g, vblocks, role, short_refs;
 };
 
 template <bool kGeneric>
@@ -2088,169 +2093,155 @@ __global__ void __launch_bounds__(kBlock) RowUpdateKernel(RowArgs a) {
   FinishBlock(st, ctrl, a.bounds, write);
 }
 
-// CSR packets keep one tile of 8,192 products between two barriers, four
-// blocks a CU: with BlockRowSum's two tiles 43,000 references of dim 64 took 107
-// us a call instead of 122, but 120,000 references of dim 256 310 instead of
-// 263, and without long rows 63,000 of dim 64 88 instead of 83.
-constexpr uint32_t kCsrTile = 8192;  // floats of a staged tile
-
-// `acc` plus references [0, count) of column c0 + threadIdx.x (`acc` when that
-// lies past the dimension; vector shapes: c0 = 0, dim <= 256).  `ok` turns
-// false in any thread that met a reference of no gradient row.  Called by the whole
-// block; `tile` holds kCsrTile floats.
-template <bool kVec>
-__device__ __forceinline__ float CsrRowSum(float* tile, const CsrRefs& refs, uint32_t count, uint32_t dim,
-                                             uint32_t c0, float acc, bool& ok) {
-  constexpr uint32_t kLongLoads = kVec ? 8 : 16;
-  const uint32_t width = kVec ? dim / 4 : min(dim - c0, kBlock);  // elements of a reference
-  uint32_t log2g = 2;                                             // lanes of a reference
-  while ((1u << log2g) < width) ++log2g;
-  const uint32_t pitch = kVec ? dim : width, cols = pitch;
-  const uint32_t per_step = kBlock >> log2g, tile_refs = kLongLoads * per_step;
-  const uint32_t sub = threadIdx.x >> log2g, e = threadIdx.x & ((1u << log2g) - 1);
-  const bool active = e < width;
-  const uint32_t at = active ? (kVec ? e * 4 : c0 + e) : (kVec ? 0u : c0);
-  float4 x[kLongLoads];
-  float scale[kLongLoads];
-  CsrRefs::Word w[kLongLoads];
-  // References past the row's end repeat its last one and are not added.
-  auto load_words = [&](uint32_t base) {
-#pragma unroll
-    for (uint32_t k = 0; k < kLongLoads; ++k) w[k] = refs.Load(min(base + k * per_step + sub, count - 1));
-  };
-  auto load_rows = [&]() {
-    const float* src[kLongLoads];
-#pragma unroll
-    for (uint32_t k = 0; k < kLongLoads; ++k) src[k] = refs.Source(w[k], at, scale[k], ok);
-#pragma unroll
-    for (uint32_t k = 0; k < kLongLoads; ++k) {
-      if constexpr (kVec) x[k] = Load4(src[k]);
-      else x[k].x = LoadF(src[k]);
-    }
-  };
-  load_words(0);
-  load_rows();
-  load_words(tile_refs);
-  for (uint32_t base = 0; base < count; base += tile_refs) {
-    LdsBarrier();  // the tile before has been added
-    if (active) {
-#pragma unroll
-      for (uint32_t k = 0; k < kLongLoads; ++k) {
-        float* to = tile + (k * per_step + sub) * pitch + (kVec ? e * 4 : e);
-        if constexpr (kVec)
-          *reinterpret_cast<float4*>(to) =
-              make_float4(x[k].x * scale[k], x[k].y * scale[k], x[k].z * scale[k], x[k].w * scale[k]);
-        else
-          *to = x[k].x * scale[k];
-      }
-    }
-    load_rows();
-    load_words(base + 2 * tile_refs);
-    LdsBarrier();
-    if (threadIdx.x < cols) {
-      const uint32_t n = min(tile_refs, count - base);
-      const float* col = tile + threadIdx.x;
-      uint32_t r = 0;
-      for (; r + 16 <= n; r += 16) {
-        float v[16];
-#pragma unroll
-        for (uint32_t k = 0; k < 16; ++k) v[k] = col[(r + k) * pitch];
-#pragma unroll
-        for (uint32_t k = 0; k < 16; ++k) acc = acc + v[k];
-      }
-      for (; r < n; ++r) acc = acc + col[r * pitch];
-    }
-  }
-  return acc;
-}
-
+// Rows of more references than this are summed by a block each.  A large packet
+// has groups enough for longer rows (200,000 references in rows of 33, dim 64:
+// 25 us with 64, 49 with 32; of 300, 28 both ways), a small one waits for them
+// (200 mean bags, dim 128, the longest row 182 references: 25 us with 64, 22
+// with 32).
+constexpr uint64_t kCsrLargeRefs = 1ull << 16;
+constexpr uint32_t CsrShortRefs(uint64_t references) { return references >= kCsrLargeRefs ? 64u : 32u; }
 constexpr uint64_t kCsrPiece = 1ull << 30;  // references of one BlockRowSum (it counts in 32 bits)
 
-// CSR rows.  Row r belongs to virtual block r % vblocks: a packet lists its
-// rows in first-occurrence order, so its long rows crowd at its start, and
-// neighbours go to different blocks.  A row of up to kBlockRowRefs references
-// takes one group, four gradient rows in flight; the block sums a longer one
-// (4,099 mean bags, 43,000 references of 11,900 rows of dim 64, the longest
-// row 3,900: one group a row, one reference in flight, 768 us; 85 us so).
+// CSR rows, a group of 2^log2g lanes a row (kGeneric: a wavefront over scalar
+// columns), four gradient rows in flight; rows of more than
+// short_refs references are left out when `short_only`.
 template <bool kGeneric>
-__global__ void __launch_bounds__(kBlock) CsrUpdateKernel(RowArgs a) {
-  __shared__ TableDesc s_t[1];
-  __shared__ uint32_t s_mode;
-  __shared__ __align__(16) float s_tile[kCsrTile];
-  Control* ctrl = a.ctrl;
-  const GuardInputs in = LoadGuard(ctrl);
-  if (threadIdx.x == 0) s_t[0] = a.t;
-  bool write = false;
-  if (!LaunchGate(ctrl, in, s_t, a.gs, a.role, &s_mode, write)) return;
+__device__ __forceinline__ void CsrShortRows(const RowArgs& a, bool short_only, bool write, RowStats& st) {
   const TableDesc T = a.t;
   const uint32_t dim = T.dim;
   const uint32_t G = kGeneric ? kWave : (1u << a.log2g);
   const uint32_t lig = threadIdx.x & (G - 1);
   const uint32_t gid = threadIdx.x / G, ngroups = kBlock / G;
-  RowStats st;
   for (uint32_t vb = blockIdx.x; vb < a.vblocks; vb += gridDim.x) {
-    const uint64_t r = uint64_t(gid) * a.vblocks + vb;
-    bool ok = true;  // the gradient scan has checked every source
-    if (r < a.rows) {
-      const uint64_t slot = a.slots[r], b = a.offsets[r], e = a.offsets[r + 1];
-      const uint32_t cnt = e > b ? uint32_t(min<uint64_t>(e - b, kBlockRowRefs + 1)) : 0u;
-      const CsrRefs refs{a.sources + b, a.scales + b, a.src, dim};
-      if (cnt > kBlockRowRefs) {
-        // below
-      } else if (!kGeneric) {
-        const uint32_t c = lig * 4;
-        const bool active = c < dim;
-        const uint32_t cl = active ? c : 0;
-        float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (uint32_t k = 0; k < cnt; k += 4) {
-          float4 x[4];
-          float s[4];
-          CsrRefs::Word w[4];
+    const uint64_t r = uint64_t(vb) * ngroups + gid;
+    if (r >= a.rows) continue;
+    const uint64_t slot = a.slots[r], b = a.offsets[r], e = max(a.offsets[r + 1], b);
+    if (short_only && e - b > a.short_refs) continue;  // (CsrTailKernel)
+    if (!kGeneric) {
+      const uint32_t c = lig * 4;
+      const bool active = c < dim;
+      float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
+      for (uint64_t j = b; j < e; j += 4) {
+        float4 x[4];
+        float s[4];
+        uint64_t source[4];
 #pragma unroll
-          for (uint32_t q = 0; q < 4; ++q) w[q] = refs.Load(min(k + q, cnt - 1));
-#pragma unroll
-          for (uint32_t q = 0; q < 4; ++q) x[q] = Load4(refs.Source(w[q], cl, s[q], ok));
-#pragma unroll
-          for (uint32_t q = 0; q < 4; ++q)
-            if (k + q < cnt) Accumulate4(g, x[q], s[q]);
+        for (uint32_t q = 0; q < 4; ++q) {
+          const bool mine = j + q < e;
+          source[q] = mine ? a.sources[j + q] : 0ull;
+          s[q] = mine ? a.scales[j + q] : 0.f;
         }
-        if (active) AdamRow4(T, slot, c, g, write, st);
-      } else {
-        for (uint32_t c = lig; c < dim; c += kWave) {
-          float g = 0.f;
-          for (uint32_t k = 0; k < cnt; k += 8) {
-            float x[8], s[8];
-            CsrRefs::Word w[8];
 #pragma unroll
-            for (uint32_t q = 0; q < 8; ++q) w[q] = refs.Load(min(k + q, cnt - 1));
+        for (uint32_t q = 0; q < 4; ++q)
+          x[q] = j + q < e && active ? Load4(a.src + source[q] * dim + c) : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-            for (uint32_t q = 0; q < 8; ++q) x[q] = LoadF(refs.Source(w[q], c, s[q], ok));
-#pragma unroll
-            for (uint32_t q = 0; q < 8; ++q)
-              if (k + q < cnt) g = g + x[q] * s[q];
-          }
-          AdamRow1(T, slot, c, g, write, st);
-        }
+        for (uint32_t q = 0; q < 4; ++q)
+          if (j + q < e) Accumulate4(g, x[q], s[q]);
       }
-    }
-    // The block's long rows, one after another (uniform over the block).
-    for (uint32_t i = 0; i < ngroups; ++i) {
-      const uint64_t row = uint64_t(i) * a.vblocks + vb;
-      if (row >= a.rows) break;
-      const uint64_t b = a.offsets[row], e = a.offsets[row + 1];
-      if (e <= b || e - b <= kBlockRowRefs) continue;
-      const uint64_t slot = a.slots[row];
-      for (uint32_t c0 = 0; c0 < dim; c0 += kBlock) {
+      if (active) AdamRow4(T, slot, c, g, write, st);
+    } else {
+      for (uint32_t c = lig; c < dim; c += kWave) {
         float g = 0.f;
-        for (uint64_t at = b; at < e; at += kCsrPiece)
-          g = CsrRowSum<!kGeneric>(s_tile, CsrRefs{a.sources + at, a.scales + at, a.src, dim},
-                                     uint32_t(min(e - at, kCsrPiece)), dim, c0, g, ok);
-        const uint32_t c = c0 + threadIdx.x;
-        if (c < dim) AdamRow1(T, slot, c, g, write, st);
+        uint64_t j = b;
+        for (; j + 4 <= e; j += 4) {
+          float x[4], s[4];
+#pragma unroll
+          for (uint32_t q = 0; q < 4; ++q) {
+            s[q] = a.scales[j + q];
+            x[q] = LoadF(a.src + a.sources[j + q] * dim + c);
+          }
+#pragma unroll
+          for (uint32_t q = 0; q < 4; ++q) g = g + x[q] * s[q];
+        }
+        for (; j < e; ++j) g = g + LoadF(a.src + a.sources[j] * dim + c) * a.scales[j];
+        AdamRow1(T, slot, c, g, write, st);
       }
     }
   }
+}
+
+// CSR rows of more than short_refs references, a block a unit of columns.  A packet lists its rows in first-occurrence order,
+// so its long rows crowd at its start: neighbours (groups of 2^spread_bits of
+// them, one in packets of up to kSpreadRows rows) go to different blocks.
+constexpr uint64_t kSpreadRows = 1ull << 18;
+struct CsrLongShared {
+  uint64_t rows[kBlock];
+  uint32_t count[3];
+  RowSumShared sum;
+};
+template <bool kGeneric>
+__device__ __forceinline__ bool CsrLongRows(const RowArgs& a, CsrLongShared& sh, RowStats& st) {
+  const TableDesc T = a.t;
+  const uint32_t dim = T.dim, slices = (dim + kLongColumns - 1) / kLongColumns;
+  const uint32_t slice = blockIdx.x % slices, c0 = slice * kLongColumns, part = blockIdx.x / slices, parts = gridDim.x / slices;
+  const uint32_t spread = a.rows <= kSpreadRows ? 0u : 3u;
+  bool found = false;
+  if (threadIdx.x == 0) sh.count[0] = 0;
+  __syncthreads();
+  uint32_t turn = 0;
+  for (uint64_t first = 0; first < a.rows; first += uint64_t(kBlock) * parts, turn = turn == 2 ? 0 : turn + 1) {
+    const uint64_t piece = (threadIdx.x >> spread) * uint64_t(parts) + part;
+    const uint64_t r = first + (piece << spread) + (threadIdx.x & ((1u << spread) - 1));
+    if (r < a.rows) {
+      const uint64_t b = a.offsets[r], e = a.offsets[r + 1];
+      if (e > b && e - b > a.short_refs) sh.rows[atomicAdd(&sh.count[turn], 1u)] = r;
+    }
+    if (threadIdx.x == 0) sh.count[turn == 2 ? 0 : turn + 1] = 0;  // (three in turn: one is still read)
+    __syncthreads();
+    const uint32_t rows = sh.count[turn];
+    found = found || rows;
+    for (uint32_t i = 0; i < rows; ++i) {
+      const uint64_t row = sh.rows[i], b = a.offsets[row], e = a.offsets[row + 1];
+      float g = 0.f;
+      bool ok = true;  // the gradient scan has checked every source
+      for (uint64_t at = b; at < e; at += kCsrPiece)
+        g = BlockRowSum<!kGeneric>(sh.sum, CsrRefs{a.sources + at, a.scales + at, a.src, dim},
+                                   uint32_t(min(e - at, kCsrPiece)), dim, c0, g, ok);
+      const uint32_t c = c0 + threadIdx.x;
+      if (threadIdx.x < kLongColumns && c < dim) AdamRow1(T, a.slots[row], c, g, true, st);
+    }
+  }
+  return found;
+}
+
+// The update of a CSR packet decides; the fused one leaves long rows to the
+// tail, the validate-only one looks at every row.
+template <bool kGeneric>
+__global__ void __launch_bounds__(kBlock) CsrUpdateKernel(RowArgs a) {
+  __shared__ TableDesc s_t[1];
+  __shared__ uint32_t s_mode;
+  Control* ctrl = a.ctrl;
+  const GuardInputs in = LoadGuard(ctrl);
+  if (threadIdx.x == 0) s_t[0] = a.t;
+  bool write = false;
+  if (!LaunchGate(ctrl, in, s_t, a.gs, kDecide, &s_mode, write)) return;
+  RowStats st;
+  CsrShortRows<kGeneric>(a, write, write, st);
   FinishBlock(st, ctrl, a.bounds, write);
+}
+
+// After it: the long rows of a fused update, every row of a checked one that
+// found nothing.  (In one kernel with the short rows, the tile's LDS and the
+// registers of the long ones cost a packet of 200,000 rows of one reference of
+// dim 16 more than half its rate, 46 -> 107 us, and rows of 33 references, one
+// block's one after another, 43 -> 184.)
+template <bool kGeneric>
+__global__ void __launch_bounds__(kBlock) CsrTailKernel(RowArgs a) {
+  __shared__ CsrLongShared sh;
+  Control* ctrl = a.ctrl;
+  const uint32_t mode = ctrl->mode, status = ctrl->status;
+  if (mode == kReject) return;
+  RowStats st;
+  if (mode == kChecked) {
+    if (status & (kErrorBits | EPS_HIP_STATUS_STALLED)) {
+      if (blockIdx.x == 0 && threadIdx.x == 0) ReportStatus(ctrl, EPS_HIP_STATUS_REJECTED);
+      return;
+    }
+    CsrShortRows<kGeneric>(a, true, true, st);
+  }
+  const bool found = CsrLongRows<kGeneric>(a, sh, st);
+  if (!found && mode != kChecked) return;
+  FinishBlock(st, ctrl, a.bounds, true);
 }
 
 // ---------------------------------------------------------------------------
@@ -2933,8 +2924,20 @@ static int RunRows(const eps_hip_table* table, const eps_hip_optimizer* optimize
   const uint64_t vb = (rows + groups - 1) / groups;
   if (vb > 0xffffffffull) return Fail(EPS_HIP_CAPACITY_EXCEEDED, "too many rows");
   a.vblocks = uint32_t(vb);
-  auto kernel = offsets ? (generic ? CsrUpdateKernel<true> : CsrUpdateKernel<false>)
-                        : (generic ? RowUpdateKernel<true> : RowUpdateKernel<false>);
+  if (offsets) {
+    a.short_refs = CsrShortRefs(references);
+    hipLaunchKernelGGL(generic ? CsrUpdateKernel<true> : CsrUpdateKernel<false>, dim3(a.vblocks), dim3(kBlock), 0, s, a);
+    EPS_HIP_LAUNCHED("csr update");
+    // (Whole turns of the column units.)
+    const uint32_t slices = (table->dim + kLongColumns - 1) / kLongColumns;
+    const uint64_t most = rows >= kTailRows ? 2 * kTailGrid : kTailGrid;
+    const uint64_t parts = std::min<uint64_t>(rows, std::max<uint64_t>(most / slices, 1));
+    hipLaunchKernelGGL(generic ? CsrTailKernel<true> : CsrTailKernel<false>, dim3(unsigned(parts * slices)), dim3(kBlock),
+                       0, s, a);
+    EPS_HIP_LAUNCHED("csr update (long rows, checked apply)");
+    return EPS_HIP_OK;
+  }
+  auto kernel = generic ? RowUpdateKernel<true> : RowUpdateKernel<false>;
   a.role = kDecide;
   hipLaunchKernelGGL(kernel, dim3(a.vblocks), dim3(kBlock), 0, s, a);
   EPS_HIP_LAUNCHED("row update");

@@ -13,27 +13,16 @@ pytestmark = pytest.mark.gpu
 F32 = np.float32
 
 
-def block_lengths(dim):
+def block_lengths(dim, widest=1 << 16):
     """Row lengths around the hand-over to the block, its tiles (4,096 products of 16-byte loads, 2,048 of scalar
     ones, a tile row the next power of two of the columns) and its groups of 128 references."""
-    pitch = 32 if dim % 4 == 0 else 16
+    vector = dim % 4 == 0 and dim <= widest
+    pitch = 32 if vector else 16
     while pitch < min(dim, 128):
         pitch *= 2
-    tile = (4096 if dim % 4 == 0 else 2048) // pitch
+    tile = (4096 if vector else 2048) // pitch
     edges = [tile - 1, tile, tile + 1, 2 * tile - 1, 2 * tile, 3 * tile + 1, 127, 128, 129, 255, 256, 257]
     return [1, 2, 4, 5, 8, 9, 31, 32, 33, 48, 49] + sorted({max(e, 33) for e in edges})
-
-
-def csr_lengths(dim):
-    """Row lengths around the hand-over to the block of a CSR packet, and its tiles."""
-    vector = dim % 4 == 0 and dim <= 256
-    width = dim // 4 if vector else min(dim, 256)
-    lanes = 4
-    while lanes < width:
-        lanes *= 2
-    tile = (8 if vector else 16) * (256 // lanes)
-    return [1, 2, 4, 5, 8, 9, 31, 32, 33, 48, 49] + [max(tile + k, 33) for k in (-1, 0, 1)] + \
-        [max(2 * tile, 33), 2 * tile + 7, 3 * tile + 1]
 
 
 def feature_of(W, rng, dim, lengths, rows):
@@ -151,37 +140,52 @@ def test_checked_apply_of_long_rows(torch_gpu, pkg, dims):
     assert all(np.array_equal(a, b) for a, b in zip(*states))
 
 
-@pytest.mark.parametrize("dim", [4, 64, 100, 256, 3, 50, 300])
-def test_compact_long_rows(torch_gpu, pkg, dim):
-    torch, W, H = torch_gpu, pkg.workloads, pkg.eps_hip
-    rng = np.random.default_rng(2000 + dim)
-    spec = W.TableSpec(0, dim, 4000, seed=5)
-    # An empty row, the edges, and enough short rows for several virtual blocks.
-    lengths = np.array([0] + csr_lengths(dim) + list(rng.integers(0, 7, 700)))
+def check_compact(torch, W, H, dim, lengths, rng, table_rows, checked=False):
+    spec = W.TableSpec(0, dim, table_rows, seed=5)
+    lengths = np.asarray(lengths)
     rows, count = len(lengths), 300
     slots = rng.permutation(spec.rows)[:rows]
     offsets = np.concatenate([[0], np.cumsum(lengths)]).astype(np.uint64)
     sources = rng.integers(0, count, int(offsets[-1])).astype(np.uint64)
     scales = rng.random(len(sources)).astype(F32)
     values = rng.normal(0, 1e-2, (count, dim)).astype(F32)
-    print(f"case: dim={dim} rows={rows} references={len(sources)}", flush=True)
+    print(f"case: dim={dim} rows={rows} references={len(sources)} checked={checked}", flush=True)
     shard = H.DeviceShard(torch, [spec])
     shard.init_rows()
+    if checked:  # a bound that the guard cannot prove safe: validated first, then applied
+        shard.bounds.view(torch.float32)[0] = 2e30
     at = torch.from_numpy(slots).cuda()
     before = shard.read_rows(0, at).cpu().numpy().reshape(rows, 3, dim)
     cuda = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
     status = shard.adam_compact(0, at, cuda(offsets.view(np.int64)), cuda(sources.view(np.int64)), cuda(scales),
                                 cuda(values))
-    assert status & H.STATUS_ERRORS == 0, f"{status:#x}"
+    assert status & H.STATUS_ERRORS == 0 and bool(status & H.STATUS_CHECKED_PATH) == checked, f"{status:#x}"
     g = np.zeros((rows, dim), F32)
-    for r in range(rows):
-        for j in range(int(offsets[r]), int(offsets[r + 1])):
-            g[r] = g[r] + values[sources[j]] * scales[j]
+    for j in range(int(lengths.max())):  # reference j of every row that has one
+        live = np.flatnonzero(lengths > j)
+        r = offsets[live].astype(np.int64) + j
+        g[live] = g[live] + values[sources[r].astype(np.int64)] * scales[r][:, None]
     rc, w, m, v = oracle.adam_rows_ctx(before[:, 0], before[:, 1], before[:, 2], g, spec.beta1, spec.beta2, spec.eps,
                                        spec.lr, spec.b1p, spec.b2p)
     assert rc == 0
     got = shard.read_rows(0, at).cpu().numpy().reshape(rows, 3, dim)
     assert_close(got, np.stack([w, m, v], 1), f"compact dim={dim}", strict_ulp=0)
+
+
+@pytest.mark.parametrize("checked", [False, True])
+@pytest.mark.parametrize("dim", [4, 64, 100, 256, 3, 50, 300, 514])
+def test_compact_long_rows(torch_gpu, pkg, dim, checked):
+    # An empty row, the edges, and enough short rows for several blocks.
+    rng = np.random.default_rng(2000 + dim)
+    lengths = [0] + block_lengths(dim, 256) + list(rng.integers(0, 7, 700))
+    check_compact(torch_gpu, pkg.workloads, pkg.eps_hip, dim, lengths, rng, 4000, checked)
+
+
+def test_compact_many_rows(torch_gpu, pkg):
+    """More rows than are looked at one by one for long ones, the long ones first and last."""
+    rng = np.random.default_rng(2100)
+    lengths = np.concatenate([block_lengths(8), rng.integers(0, 3, 290_011), [40, 33, 1, 700]])
+    check_compact(torch_gpu, pkg.workloads, pkg.eps_hip, 8, lengths, rng, 400_000)
 
 
 @pytest.mark.parametrize("dim", [4, 16, 64, 256, 6, 33, 260, 301])
