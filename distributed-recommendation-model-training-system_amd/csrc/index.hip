@@ -45,7 +45,12 @@ __device__ __forceinline__ uint64_t Spread(uint64_t k) {  // a 64-bit finaliser 
 // wavefront takes as many as its longest lane; neighbours share a cache line.
 // Evict, admit and resolve 4,096, 4,096 and 210,000 keys of an index of a million:
 // one bucket at a time 150 us with the row moves (33 of them the index), four 144.
+// An insert of kBulkInsert keys or more fills the chip: its bound is the
+// requests, and it loads one (16.8 M keys into an index of 33.6 M buckets: 4.92
+// ms with four, 4.66 with one; a million 301 us and 298, half a million 130 and
+// 132).
 constexpr uint32_t kRun = 4;
+constexpr uint64_t kBulkInsert = 1ull << 20;
 
 // The kRun buckets from `at` on (around the end; more than once in an index of
 // fewer).
@@ -76,6 +81,8 @@ __device__ __forceinline__ bool Find(const Bucket* b, uint64_t mask, uint64_t ke
   return false;
 }
 
+// (kBuckets buckets loaded at once.)
+template <uint32_t kBuckets>
 __global__ void InsertKernel(Bucket* b, uint64_t mask, const uint64_t* keys, const uint64_t* slots,
                              uint64_t count, uint32_t* status) {
   for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < count;
@@ -83,14 +90,14 @@ __global__ void InsertKernel(Bucket* b, uint64_t mask, const uint64_t* keys, con
     const uint64_t key = keys[i], slot = slots[i];
     uint64_t at = Spread(key) & mask;
     bool placed = false;
-    for (uint64_t probes = 0; probes <= mask && !placed; probes += kRun, at = (at + kRun) & mask) {
+    for (uint64_t probes = 0; probes <= mask && !placed; probes += kBuckets, at = (at + kBuckets) & mask) {
       // What a bucket holds may be old by the time it is claimed: the swap then
       // fails, since in one launch a free bucket only ever fills.
-      uint64_t seen[kRun];
+      uint64_t seen[kBuckets];
 #pragma unroll
-      for (uint32_t q = 0; q < kRun; ++q) seen[q] = b[(at + q) & mask].slot;
+      for (uint32_t q = 0; q < kBuckets; ++q) seen[q] = b[(at + q) & mask].slot;
 #pragma unroll
-      for (uint32_t q = 0; q < kRun; ++q) {
+      for (uint32_t q = 0; q < kBuckets; ++q) {
         if (placed || (seen[q] != kEmpty && seen[q] != kGone)) continue;
         Bucket* const to = b + ((at + q) & mask);
         unsigned long long* word = reinterpret_cast<unsigned long long*>(&to->slot);
@@ -179,8 +186,8 @@ int eps_hip_index_insert(void* index, uint64_t capacity, const uint64_t* keys, c
   EPS_HIP_TRY(CheckIndex(index, capacity));
   if (!count) return EPS_HIP_OK;
   if (!keys || !slots) return Fail(EPS_HIP_INVALID_ARGUMENT, "null index insert buffers");
-  hipLaunchKernelGGL(InsertKernel, dim3(Blocks(count)), dim3(kBlock), 0, AsStream(stream),
-                     static_cast<Bucket*>(index), capacity - 1, keys, slots, count, status);
+  hipLaunchKernelGGL(count >= kBulkInsert ? InsertKernel<1> : InsertKernel<kRun>, dim3(Blocks(count)), dim3(kBlock), 0,
+                     AsStream(stream), static_cast<Bucket*>(index), capacity - 1, keys, slots, count, status);
   EPS_HIP_LAUNCHED("index insert");
   return EPS_HIP_OK;
 }

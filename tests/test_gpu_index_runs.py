@@ -1,5 +1,6 @@
-"""Key index with buckets probed four at a time: indexes smaller than a run, runs
-around the end, an index without an empty bucket, and keys that are not in it."""
+"""Key index with buckets probed four at a time (inserts of 2^20 keys and more:
+one): indexes smaller than a run, runs around the end, an index without an empty
+bucket, and keys that are not in it."""
 import ctypes as C
 
 import numpy as np
@@ -8,7 +9,8 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("capacity,count", [(2, 1), (2, 2), (4, 3), (8, 8), (256, 250), (1024, 1024), (1 << 16, 30_011)])
+@pytest.mark.parametrize("capacity,count", [(2, 1), (2, 2), (4, 3), (8, 8), (256, 250), (1024, 1024), (1 << 16, 30_011),
+                                            (1 << 21, 1 << 20)])
 def test_insert_remove_resolve(torch_gpu, pkg, capacity, count):
     torch, H = torch_gpu, pkg.eps_hip
     lib = H.lib()
