@@ -455,7 +455,11 @@ __device__ void FinishBlock(const RowStats& st, Control* ctrl, Bounds* bounds, b
 // 64 without long rows 320 -> 306.  Tiles of 8,192 products add 13 ns a
 // reference of dim 64 instead of 16, but leave two blocks a CU: 387 us for
 // those eight tables.
-constexpr uint32_t kBlockRowRefs = 32;   // rows with more references are summed by the block
+// Rows with more references are summed by the block.  (Reduce of six tables of
+// dims 10 to 300, 10,600 references each: 95 us with 16, 100 with 32, 107 with
+// 64; 200,000 references of dim 64 in rows of 24 133, 123 and 123, in rows of 48
+// 112, 112 and 129.)
+constexpr uint32_t kBlockRowRefs = 32;
 constexpr uint32_t kLongTile = 4096;     // floats of a staged tile (of two)
 // Columns of a row that one block sums; wider rows are units of as many, on
 // different blocks.  (43,000 references of dim 300, Zipf of 1.05, pushed: units

@@ -509,8 +509,10 @@ __global__ void InitRowsKernel(float* state, uint32_t dim, uint64_t first, uint6
 // From pinned host memory the host link bounds it, and the link is slower with
 // more reads waiting on it than fill it: 4,096 rows of dim 64 (3.1 MB) take 128
 // us with 8 blocks of 16-byte loads, 68 with 16, 60 with 32 or 64, 64 with 256
-// and 79 with 768, a thread a load (a copy of that size 69).  Loads of 4 bytes
-// keep a thread a load.
+// and 79 with 768, a thread a load (a copy of that size 69).  The other widths
+// and counts gain as much or nothing: 65,536 rows of dim 4 77 -> 59, 262,144 262
+// -> 223, 1,024 6.5 either way; 16,384 rows of dim 256 957 -> 879.  Loads of 4
+// bytes keep a thread a load.
 constexpr unsigned kHostReadGrid = 64;
 __global__ void ScatterRowsKernel(float* state, uint32_t dim, const uint64_t* slots,
                                   const float* packed, uint64_t count, Bounds* bounds) {

@@ -61,7 +61,10 @@ constexpr uint32_t kProbes = 128;        // offsets probed in a round of a block
 // Largest number of keygen tiles of a table whose counts a pass's blocks add
 // up themselves (each thread one digit, eight loads in flight).  Above it one
 // more launch adds them up per table (CountSumKernel), and the first pass
-// looks back like the others.
+// looks back like the others: 131,000 references on a table of a million rows
+// take 43 us with the blocks adding and 54 with the launch, 26 tables of 43,000
+// 67 and 77.  Past 32 tiles it depends: 200,000 on one table 48 and 63, but
+// 400,000 on each of four 123 and 110.
 constexpr uint32_t kDirectTiles = 32;
 
 struct PrepFeature {
@@ -421,7 +424,7 @@ struct SortArgs {
   // Per segment (a table with occurrences, by key index): first element,
   // first keygen tile (and the ends), key index.
   uint32_t seg_begin[EPS_HIP_MAX_TABLES], seg_tile[EPS_HIP_MAX_TABLES + 1], seg_key[EPS_HIP_MAX_TABLES];
-  uint32_t segments, tiles, shift, bits, digits, pass, passes, count_tiles, sentinel;
+  uint32_t segments, shift, bits, digits, pass, passes, count_tiles, sentinel;
   uint32_t direct;  // counts are added up by the block (no CountSumKernel ran)
   uint32_t class_key[kClasses + 1];  // first table key index of each class (+ table count)
   const uint16_t* counts;
@@ -1367,7 +1370,6 @@ int Prepare(const eps_hip_table* tables, uint32_t table_count, const eps_hip_pus
     SortArgs a = p == 0 ? first : later;
     const uint32_t grid = p == 0 ? blocks : later_blocks;
     a.segments = segments;
-    a.tiles = grid;
     a.shift = plan.shift[p];
     a.bits = plan.bits[p];
     a.digits = args.digits;

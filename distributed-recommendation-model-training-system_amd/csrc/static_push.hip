@@ -7,7 +7,7 @@
 // until the process ends) at its own address, found once per device with
 // hipGetSymbolAddress; kernels get that address, never the symbol.  Calls on
 // one GPU share the array, so calls that overlap on one GPU race; each call's
-// preparation clears what must start at zero (with a fill kernel).  Every
+// preparation clears what must start at zero (in its own kernels).  Every
 // kernel of a call runs on the caller's stream (no side stream or event), and
 // the only runtime calls besides launches are the first call's symbol lookup
 // per device, so a call can be captured in a graph once that lookup is done.

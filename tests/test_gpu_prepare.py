@@ -71,6 +71,20 @@ def test_occurrence_counts(torch_gpu, pkg, occurrences, weighted):
     check(torch, W, H, specs, [feature(W, rng, specs, 0, 0, occurrences, pooling, holes=0.1)])
 
 
+@pytest.mark.parametrize("pooled,sequences,occurrences", [(32, 0, 4096), (32, 0, 4097), (16, 3, 2049), (0, 32, 4096)])
+def test_many_features(torch_gpu, pkg, pooled, sequences, occurrences):
+    """As many features as a push holds, over three tables, in one block and in tiles."""
+    torch, W, H = torch_gpu, pkg.workloads, pkg.eps_hip
+    rng = np.random.default_rng(pooled + occurrences)
+    specs = [W.TableSpec(i, d, 900, seed=20 + i) for i, d in enumerate([4, 64, 10])]
+    count = pooled + sequences
+    share = [occurrences // count + (i < occurrences % count) for i in range(count)]
+    feats = [feature(W, rng, specs, i % 3, i, share[i],
+                     W.SEQUENCE if i >= pooled else [W.SUM, W.MEAN, W.WEIGHTED_SUM][i % 3]) for i in range(count)]
+    print(f"case: {pooled} pooled features, {sequences} sequences, {occurrences} occurrences", flush=True)
+    check(torch, W, H, specs, feats)
+
+
 @pytest.mark.parametrize("empty", [0, 5000, 8000, 9000])
 def test_empty_bags_beside_the_staged_offsets(torch_gpu, pkg, empty):
     torch, W, H = torch_gpu, pkg.workloads, pkg.eps_hip
