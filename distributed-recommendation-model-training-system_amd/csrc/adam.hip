@@ -446,15 +446,13 @@ __device__ void FinishBlock(const RowStats& st, Control* ctrl, Bounds* bounds, b
 // LDS reads a step ahead of its adds.  The sum is the group loop's, bit for
 // bit: acc = acc + src * scale, in order, from +0 (products past the row's end
 // are staged as -0.0f, the identity).  What bounds it is the adding waves:
-// their adds, their share of the staging and a barrier per tile.  Rows past
-// 256 columns take 16-byte loads too, where their alignment allows them.
-// Reduce of six tables of dims 10 to 300, 10,600 references each, the longest
-// rows ~1,000: 328 -> 202 us a dedup and reduce (4-byte loads, one tile of 16
-// references in flight, 80 ns a reference of dim 300 before); four tables of
-// dim 128, 63,000 references each, the longest ~15 %: 486 -> 416; eight of dim
-// 64 without long rows 320 -> 306.  Tiles of 8,192 products add 13 ns a
-// reference of dim 64 instead of 16, but leave two blocks a CU: 387 us for
-// those eight tables.
+// their adds, their share of the staging and a barrier per tile: 16 ns a
+// reference of dim 64 (a tile of 8,192 products 13, but two blocks a CU).  Rows
+// past 256 columns take 16-byte loads too, where their alignment allows them.
+// Dedup and reduce of six tables of dims 10 to 300, 10,600 references each, the
+// longest rows ~1,000: 2,057 us with a group a row, 328 with 4-byte loads and
+// one tile of 16 references in flight, 202 so, 168 with the short rows launched
+// apart and units of 128 columns (below).
 // Rows with more references are summed by the block.  (Reduce of six tables of
 // dims 10 to 300, 10,600 references each: 95 us with 16, 100 with 32, 107 with
 // 64; 200,000 references of dim 64 in rows of 24 133, 123 and 123, in rows of 48
@@ -2052,6 +2050,8 @@ RowRunClassesKernel(VecArgs a) {
 
 // ---------------------------------------------------------------------------
 // Row driver: explicit unique rows (ApplyHost) or CSR references (ApplyCompact).
+// 43,000 references of 14,700 rows of dim 64, the longest 3,787: 751 us with a
+// group a row and one reference in flight, 75 so (short rows 14, long rows 60).
 struct RowArgs {
   TableDesc t;
   const uint64_t* slots;
@@ -2382,7 +2382,12 @@ constexpr uint64_t kLongGrid = 2048;      // grid cap of the long rows' launches
 // Grid cap of a class's short rows: six classes in one launch stay below the
 // 2^32 threads that one can have.
 constexpr uint64_t kSortedGrid = 1ull << 21;
-constexpr uint64_t kHotGrid = 512;      // two blocks per CU (LDS: four 17 KiB tiles per block)
+// Blocks of the 16- and 32-column hot-row kernels.  A CU holds one of the
+// former (87 KB of LDS) and two of the latter (68 KB).  4 x 8.4 M references:
+// 256 blocks 8.64 ms a push, 512 5.67, 1,024 5.72; the 16-column kernel takes as
+// long with any of them (65,536 pairs 67 to 68 us: its hottest row is one block
+// a unit).
+constexpr uint64_t kHotGrid = 512;
 // Blocks of the 64-column hot-row kernel beside the row kernels: enough to
 // finish the hot rows well before the row kernels do, few enough to leave
 // them most of the GPU (26 tables of ~43,000 references: 64 blocks 259 us a
