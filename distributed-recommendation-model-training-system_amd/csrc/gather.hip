@@ -198,8 +198,8 @@ __device__ __forceinline__ void PoolRows(const GatherDesc& d, GatherShared& sh, 
   // steps' loads go out together, without the rest of a batch (10,000 bags of
   // dim 258, 12.7 us as sums, 7.8 so; of dim 300, 10.4 and 7.8).
   const uint64_t first = sh.off[r] - occ_begin;
-  if (once && G * V < d.dim && r < nrows && sh.off[r + 1] - sh.off[r] == 1 && first < kIdCap &&
-      (kBuffered || sh.at64[first] != kHole)) {
+  if (once && G * V < d.dim && r < nrows && sh.off[r + 1] - sh.off[r] == 1 && sh.off[r + 1] <= occ_end &&
+      first < kIdCap && (kBuffered || sh.at64[first] != kHole)) {  // (staged, whatever the offsets)
     const uint32_t at = kBuffered ? sh.at32[first] : 0u;  // (a hole reads zeros)
     const float weight = !kWeighted ? 1.f : kBuffered && at == kBufferOutside ? 0.f : sh.weight[first];
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -284,7 +284,8 @@ __device__ __forceinline__ void PoolRows(const GatherDesc& d, GatherShared& sh, 
         __syncthreads();  // the chunk before has been added
         StageOccurrences(d, sh, chunk, n, bad);
         __syncthreads();
-        if (active && sh.off[r] < sh.off[r + 1]) add_staged(std::integral_constant<uint32_t, kGatherBatch>{}, 0u, n);
+        if (active && sh.off[r] == occ_begin && sh.off[r + 1] == occ_end)
+          add_staged(std::integral_constant<uint32_t, kGatherBatch>{}, 0u, n);
       }
     } else if (once) {
       // (Kept inside the staged entries, whatever the offsets.)
@@ -301,8 +302,8 @@ __device__ __forceinline__ void PoolRows(const GatherDesc& d, GatherShared& sh, 
       // only bag is better off with that (20,000 rows of dim 3: 0.99 ms, its
       // group alone 2.65; 500,000 of dim 64: 23, 29).
       const uint32_t entry = r * room;
-      for (uint64_t from = sh.off[r]; from < sh.off[r + 1]; from += room) {
-        const uint32_t n = uint32_t(min<uint64_t>(room, sh.off[r + 1] - from));
+      for (uint64_t from = max(sh.off[r], occ_begin); from < min(sh.off[r + 1], occ_end); from += room) {
+        const uint32_t n = uint32_t(min<uint64_t>(room, min(sh.off[r + 1], occ_end) - from));
         uint64_t idx[kOwn];
 #pragma unroll
         for (uint32_t k = 0; k < kOwn; ++k) idx[k] = d.indices[from + min(k * G + lig, n - 1)];

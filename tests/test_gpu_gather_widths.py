@@ -3,6 +3,8 @@ dimension and the buffers' alignment), of rows wider than a wavefront's
 columns, of sequence copies, of bags past what a block stages at a time and of
 sources read by 64-bit offsets, bit-exact against the oracle (sums are taken in
 occurrence order)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -109,3 +111,26 @@ def test_bags_past_the_stage_past_a_buffer_range(torch_gpu, pkg, dim, pooling):
 def test_only_holes(torch_gpu, pkg, dim, pooling):
     check(torch_gpu, pkg.workloads, pkg.eps_hip, dim, pooling, np.random.default_rng(dim), rows=60, bags=9, max_len=30,
           holes=1.0)
+
+
+@pytest.mark.parametrize("dim", [64, 258, 300, 1028, 16_385, 16_388])
+@pytest.mark.parametrize("lengths", [[1] * 40, [0, 1, 0, 3], [700, 1, 900, 1], [2000]])
+def test_occurrences_claimed_without_indices(torch_gpu, pkg, dim, lengths):
+    """Offsets that claim occurrences of a part without indices are bad indices: zeros, and the status bit."""
+    torch, H = torch_gpu, pkg.eps_hip
+    print(f"case: dim={dim} bags={len(lengths)}", flush=True)
+    source = torch.full((60, dim), 3.0, device="cuda")
+    offsets = torch.from_numpy(np.concatenate([[0], np.cumsum(lengths)])).cuda()
+    valid = torch.from_numpy(np.asarray(lengths)).cuda()
+    status = torch.zeros(1, dtype=torch.int32, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    for pooling in (H.SUM, H.MEAN, H.WEIGHTED_SUM):
+        out = torch.full((len(lengths), dim), -7.0, device="cuda")
+        part = H.GatherPart(source.data_ptr(), None, None, offsets.data_ptr(),
+                            valid.data_ptr() if pooling == H.MEAN else None, None, out.data_ptr(), dim, len(lengths),
+                            60, 0, dim, pooling)
+        status.zero_()
+        H.check(H.lib().eps_hip_gather(C.byref(part), 1, status.data_ptr(), stream))
+        torch.cuda.synchronize()
+        assert int(status) & H.STATUS_BAD_INDEX
+        assert not out.any()
